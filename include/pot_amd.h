@@ -50,6 +50,11 @@ const char* potamd_status_string(int code);
 /* Bytes of workspace needed by potamd_sinkhorn_dense. */
 size_t potamd_dense_workspace_size(int dtype, int batch, int n, int m, int rows_per_block);
 
+/* 1 if a solve of this shape keeps its cost in the register files when it is
+ * called with threads = cols_per_thread = 0, 0 if it runs on the row sweep,
+ * whose tile the caller may then choose. */
+int potamd_dense_resident(int dtype, int batch, int n, int m);
+
 /* Dense-cost Sinkhorn on `batch` problems of shape n x m sharing one reg.
  *
  * Replaces the iteration loops of

@@ -49,9 +49,10 @@ def dense_solve(M, a, b, u0, v0, reg, *, domain, order, kernel_given=False,
         bs = M.stride(0) if bstride is None else bstride
     if M.stride(-1) != 1:
         raise ValueError("cost rows must be contiguous")
-    if tile is None:
+    if tile is None and not lib.potamd_dense_resident(code, B, n, m):
         from . import autotune
         tile = autotune.lookup("f32" if code == _lib.F32 else "f64", n, m)
+    # (without a tile the library keeps a cost that fits in registers)
     T, cpt, rpb, pf = (tuple(tile) + (0,) * 4)[:4] if tile else (0, 0, 0, 0)
     ws_bytes = lib.potamd_dense_workspace_size(code, B, n, m, rpb)
     if ws_bytes == 0:

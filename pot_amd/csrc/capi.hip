@@ -59,6 +59,7 @@ struct DenseLayout {
   Ctrl* ctrl;
   int* bad;
   int* pstate;  // per-problem stop: [B] done, [B] niter, [B] status
+  char* words;  // exchange slots of the register-resident solve
   size_t bytes;
 };
 
@@ -82,6 +83,7 @@ DenseLayout carve_dense(void* ws, int dtype, int B, int n, int m, int rpb) {
   L.ctrl = c.take<Ctrl>(1);
   L.bad = c.take<int>(2);
   L.pstate = c.take<int>((size_t)3 * B);
+  L.words = c.take<char>(resident_workspace(dtype, B, n, m));
   L.bytes = c.off;
   return L;
 }
@@ -114,6 +116,11 @@ extern "C" size_t potamd_dense_workspace_size(int dtype, int batch, int n, int m
   if (batch < 1 || n < 1 || m < 1) return 0;
   const int rpb = rows_per_block > 0 ? rows_per_block : default_rpb(n);
   return carve_dense(nullptr, dtype, batch, n, m, rpb).bytes;
+}
+
+extern "C" int potamd_dense_resident(int dtype, int batch, int n, int m) {
+  if ((dtype != POTAMD_F32 && dtype != POTAMD_F64) || batch < 1 || n < 1 || m < 1) return 0;
+  return resident_fits(dtype, batch, n, m) ? 1 : 0;
 }
 
 namespace {
@@ -166,6 +173,51 @@ int dense_impl(int dtype, int domain, int order, int kernel_given, const void* M
     s2 = -kLog2e / reg;
   float s_hi, s_lo;
   split_f32(s2, &s_hi, &s_lo);
+
+  // A problem that fits the register files stays there (the caller who names
+  // a row-sweep tile gets the row sweep).
+  if (threads == 0 && cols_per_thread == 0 && resident_fits(dtype, batch, n, m)) {
+    ResidentArgs r;
+    memset(&r, 0, sizeof(r));
+    r.M = M;
+    r.ldm = ldm;
+    r.bstride = bstride;
+    r.n = n;
+    r.m = m;
+    r.B = batch;
+    r.s2 = s2;
+    r.s_hi = s_hi;
+    r.s_lo = s_lo;
+    r.logd = logd;
+    r.kernel_given = kernel_given;
+    r.row_first = order == POTAMD_ROW_FIRST;
+    r.each = each;
+    r.err_norm = err_norm;
+    r.a = a;
+    r.b = b;
+    r.u_in = r.u_out = u;
+    r.v_in = r.v_out = v;
+    r.max_iter = max_iter;
+    r.stop_thr = stop_thr;
+    r.err_hist = err_hist;
+    r.err_cap = err_cap;
+    r.errpart = L.errpart;
+    r.niters = niters;
+    r.statuses = statuses;
+    r.words = reinterpret_cast<unsigned long long*>(L.words);
+    r.ctrl = L.ctrl;
+    Ctrl got;
+    const int done =
+        resident_solve(dtype, r, L.U[0], L.V[0], static_cast<Ctrl*>(host_ctrl), s, &got);
+    if (done < 0) return POTAMD_EHIP;
+    if (done == 0) {
+      info[0] = got.niter;
+      info[1] = got.n_err;
+      info[2] = got.status;
+      info[3] = got.bad_iter;
+      return got.status;
+    }
+  }
 
   // Set-up: log2 weights, initial state, control block.
   HIP_TRY(launch_ctrl_init(L.ctrl, L.bad, s));

@@ -49,6 +49,43 @@ struct MergeArgs {
   int* pstate;          // err_norm 2: [B] done, [B] niter, [B] status
 };
 
+// Dense solve with the cost in registers (dense_resident.hip).
+struct ResidentArgs {
+  const void* M;
+  int64_t ldm, bstride;
+  int n, m, B;
+  int R, C;              // blocks of a problem: row x column blocks
+  int rbs, cbs;          // rows and columns of a block
+  double s2;
+  float s_hi, s_lo;
+  int logd, kernel_given, row_first;
+  int each;              // every problem stops on its own check
+  int err_norm;          // batch error: 0 max over problems, 1 Frobenius
+  const double* a;       // B x n
+  const double* b;       // B x m
+  const double* u_in;    // start (natural units; a resumed segment: base 2)
+  const double* v_in;
+  double* u_out;
+  double* v_out;
+  int max_iter, it0;
+  int segment, resume;   // one launch per check interval, and not its first
+  double stop_thr;
+  double* err_hist;
+  int err_cap;
+  double* errpart;       // B (segments)
+  int* niters;           // each
+  int* statuses;         // each
+  unsigned long long* words;  // exchange slots
+  int row_slot, col_slot;
+  int64_t err_slot, col_base, err_base;
+  Ctrl* ctrl;            // counter != 0: abandoned
+};
+
+bool resident_fits(int dtype, int B, int n, int m);
+size_t resident_workspace(int dtype, int B, int n, int m);
+int resident_solve(int dtype, ResidentArgs a, double* u_keep, double* v_keep, Ctrl* host_ctrl,
+                   hipStream_t s, Ctrl* out);
+
 struct ColLseArgs {
   const void* M;
   int64_t ldm, bstride;
