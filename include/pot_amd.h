@@ -136,6 +136,15 @@ int potamd_plan_dense(int dtype, int domain, int kernel_given, const void* M, in
                       int64_t pstride, double* sums, void* workspace, size_t ws_bytes,
                       void* stream);
 
+/* potamd_plan_dense with the sums chosen: `which` adds 1 for sums[0] and
+ * sums[3], 2 for sums[1], 4 for sums[2]; the others are 0.  A logarithm per
+ * element is saved for each of the last two that is left out. */
+int potamd_plan_dense_sums(int which, int dtype, int domain, int kernel_given, const void* M,
+                           int64_t ldm, int64_t bstride, int batch, int n, int m, double reg,
+                           const double* u, const double* v, const double* a, const double* b,
+                           void* P, void* logP, int64_t pstride, double* sums, void* workspace,
+                           size_t ws_bytes, void* stream);
+
 /* Batched (squared) Euclidean cost matrices.
  * Replaces ot.dist / ot.utils.euclidean_distances (ot/utils.py:270-307,
  * :465-468; clamp = 1, zero_diag when X is Y) and

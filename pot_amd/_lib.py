@@ -43,6 +43,9 @@ SIGNATURES = {
     "potamd_plan_dense": (c_int, [
         c_int, c_int, c_int, c_vp, c_i64, c_i64, c_int, c_int, c_int, c_dbl,
         c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i64, c_vp, c_vp, c_size, c_vp]),
+    "potamd_plan_dense_sums": (c_int, [
+        c_int, c_int, c_int, c_int, c_vp, c_i64, c_i64, c_int, c_int, c_int, c_dbl,
+        c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i64, c_vp, c_vp, c_size, c_vp]),
     "potamd_sinkhorn_log_batch": (c_int, [
         c_int, c_int, c_int, c_int, c_vp,    # dtype, batch, max_n, max_m, M
         c_vp, c_vp, c_vp, c_vp,              # moff, ns, ms, ldms

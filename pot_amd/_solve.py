@@ -96,10 +96,14 @@ def dense_solve(M, a, b, u0, v0, reg, *, domain, order, kernel_given=False,
                        status=info[2], bad_iter=info[3], niters=niters, statuses=statuses)
 
 
+SUM_COST, SUM_ENTROPY, SUM_KL = 1, 2, 4  # columns 0 (and 3, the mass), 1 and 2
+
+
 def plan(M, u, v, reg, *, domain, kernel_given=False, a=None, b=None,
-         want_plan=True, want_log=False, want_sums=True, batch=None, bstride=None,
-         out_dtype=None):
-    """Run potamd_plan_dense; returns (P, logP, sums) (None where not asked)."""
+         want_plan=True, want_log=False, want_sums=SUM_COST | SUM_ENTROPY | SUM_KL, batch=None,
+         bstride=None, out_dtype=None):
+    """Run potamd_plan_dense_sums; returns (P, logP, sums) (None where not
+    asked); ``want_sums`` combines the SUM_ flags (0: none)."""
     lib = _lib.load()
     dev = M.device
     code = _lib.F32 if M.dtype == torch.float32 else _lib.F64
@@ -117,14 +121,14 @@ def plan(M, u, v, reg, *, domain, kernel_given=False, a=None, b=None,
     sums = torch.empty((B, 4), dtype=torch.float64, device=dev) if want_sums else None
     ws_bytes = lib.potamd_plan_workspace_size(B, n)
     ws = _device.workspace(ws_bytes, dev)
-    rc = lib.potamd_plan_dense(
-        code, domain, int(bool(kernel_given)), _ptr(M), ldm, bs, B, n, m,
+    rc = lib.potamd_plan_dense_sums(
+        int(want_sums) or SUM_COST, code, domain, int(bool(kernel_given)), _ptr(M), ldm, bs, B, n, m,
         float(reg) if reg is not None else 1.0,
         _ptr(u.contiguous()), _ptr(v.contiguous()),
         _ptr(a) if a is not None else None, _ptr(b) if b is not None else None,
         _ptr(P), _ptr(L), n * m, _ptr(sums), _ptr(ws), ws_bytes,
         ctypes.c_void_p(_device.stream_ptr(dev)))
-    _lib.check(rc, "potamd_plan_dense")
+    _lib.check(rc, "potamd_plan_dense_sums")
     return P, L, sums
 
 

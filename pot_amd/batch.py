@@ -130,7 +130,7 @@ def _projection(K, a, b, max_iter, tol, domain, grad):
                                   stop_thr=0.0, err_norm=0)
         u, v = res1.u, res1.v
     P, L, _ = _solve.plan(Kt, u, v, None, domain=domain, kernel_given=True,
-                          want_log=domain == _lib.LOG, want_sums=False)
+                          want_log=domain == _lib.LOG, want_sums=0)
     T = ing.out(P)
     log_T = None if L is None else ing.out(L)
     return ing, res.niter, T, log_T, (ing.out(u), ing.out(v)), False
@@ -362,7 +362,9 @@ def solve_batch(M, reg, a=None, b=None, max_iter=1000, tol=1e-5, solver="log_sin
                                   max_iter=1, stop_thr=0.0, err_norm=0)
         u, v = res1.u, res1.v
 
-    P, _, sums = _solve.plan(Mt, u, v, reg, domain=domain, a=at, b=bt)
+    P, _, sums = _solve.plan(Mt, u, v, reg, domain=domain, a=at, b=bt,
+                             want_sums=_solve.SUM_COST | (_solve.SUM_KL if kl
+                                                          else _solve.SUM_ENTROPY))
     value_linear = sums[:, 0]
     value = value_linear + reg * (sums[:, 2] if kl else sums[:, 1])
     potentials = (ing.out(u), ing.out(v))

@@ -248,7 +248,8 @@ def sinkhorn_log(a, b, M, reg, numItermax=1000, stopThr=1e-9, verbose=False,
             warnings.warn(NOT_CONVERGED)
 
     P, _, sums = _solve.plan(Mt, u, v, reg, domain=_lib.LOG,
-                             want_plan=_grad_parts or not _loss_only)
+                             want_plan=_grad_parts or not _loss_only,
+                             want_sums=_solve.SUM_COST if _grad_parts or _loss_only else 0)
     out = ing.scalar(sums[0, 0].item()) if _loss_only else ing.out(P[0])
     logd = None
     if log:
@@ -293,7 +294,7 @@ def _sinkhorn_log_columns(ing, Mt, at, bt, reg, numItermax, stopThr, log, ws):
         if st == _lib.MAX_ITER:
             warnings.warn(NOT_CONVERGED)
     _, _, sums = _solve.plan(Mt, res.u, res.v, reg, domain=_lib.LOG, want_plan=False,
-                             batch=nh, bstride=0)
+                             want_sums=_solve.SUM_COST, batch=nh, bstride=0)
     out = ing.out(sums[:, 0])
     if not log:
         return out
@@ -351,6 +352,7 @@ def sinkhorn_knopp(a, b, M, reg, numItermax=1000, stopThr=1e-9, verbose=False,
 
     want_plan = _grad_parts or not (nh or _loss_only)
     P, _, sums = _solve.plan(Mt, u, v, reg, domain=_lib.SCALING, want_plan=want_plan,
+                             want_sums=_solve.SUM_COST if nh or _loss_only or _grad_parts else 0,
                              batch=B, bstride=0)
     if nh:
         out = ing.out(sums[:, 0])

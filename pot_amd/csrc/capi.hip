@@ -444,14 +444,14 @@ extern "C" size_t potamd_plan_workspace_size(int batch, int n) {
   return align_up((size_t)batch * plan_blocks(n) * 4 * sizeof(double));
 }
 
-extern "C" int potamd_plan_dense(int dtype, int domain, int kernel_given, const void* M,
+extern "C" int potamd_plan_dense_sums(int which, int dtype, int domain, int kernel_given, const void* M,
                                  int64_t ldm, int64_t bstride, int batch, int n, int m,
                                  double reg, const double* u, const double* v, const double* a,
                                  const double* b, void* P, void* logP, int64_t pstride,
                                  double* sums, void* workspace, size_t ws_bytes, void* stream) {
   if ((dtype != POTAMD_F32 && dtype != POTAMD_F64) || !M || !u || !v || batch < 1 || n < 1 ||
       m < 1 || ldm < m || (!kernel_given && domain == POTAMD_LOG && !(reg > 0.0)) ||
-      ((P || logP) && batch > 1 && pstride < (int64_t)n * m))
+      ((P || logP) && batch > 1 && pstride < (int64_t)n * m) || which < 1 || which > 7)
     return POTAMD_EINVAL;
   if (!workspace || ws_bytes < potamd_plan_workspace_size(batch, n)) return POTAMD_EWORKSPACE;
   PlanArgs pa;
@@ -470,10 +470,20 @@ extern "C" int potamd_plan_dense(int dtype, int domain, int kernel_given, const 
   pa.b = (a && b) ? b : nullptr;
   pa.P = P;
   pa.logP = logP;
-  pa.pstride = pstride;
+  pa.pstride = batch > 1 ? pstride : 0;
+  pa.which = a && b ? which : which & 3;
   pa.partial = static_cast<double*>(workspace);
   HIP_TRY(launch_plan(dtype, pa, batch, sums, static_cast<hipStream_t>(stream)));
   return 0;
+}
+
+extern "C" int potamd_plan_dense(int dtype, int domain, int kernel_given, const void* M,
+                                 int64_t ldm, int64_t bstride, int batch, int n, int m,
+                                 double reg, const double* u, const double* v, const double* a,
+                                 const double* b, void* P, void* logP, int64_t pstride,
+                                 double* sums, void* workspace, size_t ws_bytes, void* stream) {
+  return potamd_plan_dense_sums(7, dtype, domain, kernel_given, M, ldm, bstride, batch, n, m, reg,
+                                u, v, a, b, P, logP, pstride, sums, workspace, ws_bytes, stream);
 }
 
 extern "C" int potamd_sqeuclidean(int dtype, const void* X, const void* Y, int batch, int n,

@@ -110,6 +110,8 @@ struct PlanArgs {
   void* logP;        // log plan out (log domain), may be null
   int64_t pstride;   // problem stride of P / logP
   double* partial;   // B x blocks x 4
+  int which;         // sums wanted: 1 cost and mass, 2 entropy, 4 KL
+  int tx, csplit;    // log2 of the column threads; column splits of a row block
 };
 
 struct DistArgs {

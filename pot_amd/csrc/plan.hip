@@ -9,6 +9,12 @@
 //   sums[1] = sum P * log(P + 1e-16)     (-entropy_batch, _utils.py:4-22)
 //   sums[2] = sum P * log(P / (a b) + 1e-16)  (KL value, _linear.py:342-345)
 //   sums[3] = sum P
+// Bound: the plan alone reads the cost and writes P (16384^2 float32: 2.1 GB);
+// the sums are bound by the fp64 exponential and logarithms, so a logarithm is
+// taken only where its sum is asked for.
+#include <algorithm>
+
+#include "host.h"
 #include "internal.h"
 
 namespace potamd {
@@ -16,47 +22,112 @@ namespace potamd {
 constexpr int kPlanThreads = 256;
 constexpr int kPlanSums = 4;
 
-template <typename TM>
+// 2^t to 2^-33 relative (the polynomial interpolates 2^r on [-1/2, 1/2] at the
+// Chebyshev nodes of degree 8): an fp32 result is rounded as from the exact
+// value, for half the instructions of exp().
+__device__ __forceinline__ double exp2_for_f32(double t) {
+  t = t < -1100.0 ? -1100.0 : (t > 1100.0 ? 1100.0 : t);  // infinities; a NaN stays
+  const double k = rint(t), r = t - k;
+  double y = 1.5303700711365693e-05;
+  y = fma(y, r, 0.00015469729214118296);
+  y = fma(y, r, 0.0013333478473685416);
+  y = fma(y, r, 0.009618025613318034);
+  y = fma(y, r, 0.055504109063258665);
+  y = fma(y, r, 0.24022651213498092);
+  y = fma(y, r, 0.6931471805568324);
+  y = fma(y, r, 0.9999999999595618);
+  return ldexp(y, (int)k);
+}
+
+template <typename TM, int VEC>
+struct alignas(sizeof(TM) * VEC) PlanVec {
+  TM x[VEC];
+};
+
+// A thread owns VEC adjacent columns, whose v stays in registers, and walks
+// down the block's rows, four at a time in flight: 1 << A.tx column threads by
+// 256 >> A.tx row threads.  (A row at a time over 256 column threads left 3 of
+// 4 threads idle at 64 columns, read v anew for every row and waited for each
+// load: 512 plans of 64^2 took 51 us, 16384^2 float32 1464 us.)
+template <typename TM, int VEC, bool SUMS>
 __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs A) {
+  using V = PlanVec<TM, VEC>;
   const int p = blockIdx.y;
   const int n = A.n, m = A.m;
+  const int TX = 1 << A.tx, TY = kPlanThreads >> A.tx;
+  const int tx = threadIdx.x & (TX - 1), ty = threadIdx.x >> A.tx;
   const TM* Mp = static_cast<const TM*>(A.M) + (int64_t)p * A.bstride;
   const double* u = A.u + (int64_t)p * n;
   const double* v = A.v + (int64_t)p * m;
   TM* P = A.P ? static_cast<TM*>(A.P) + (int64_t)p * A.pstride : nullptr;
   TM* L = A.logP ? static_cast<TM*>(A.logP) + (int64_t)p * A.pstride : nullptr;
   const double inv_reg = A.kernel_given ? 0.0 : 1.0 / A.reg;
+  const bool logd = A.domain == kLog, given = A.kernel_given;
+  const bool ent = SUMS && A.which & 2, kl = SUMS && A.which & 4;
+  const double s2 = given ? kLog2e : -kLog2e * inv_reg;
   double s_cost = 0, s_ent = 0, s_kl = 0, s_mass = 0;
-  const int r0 = blockIdx.x * A.rpb, r1 = min(n, r0 + A.rpb);
-  for (int i = r0; i < r1; ++i) {
-    const double ui = u[i];
-    const double ai = A.a ? A.a[(int64_t)p * n + i] : 1.0;
-    for (int j = threadIdx.x; j < m; j += kPlanThreads) {
-      const double mij = (double)Mp[(int64_t)i * A.ldm + j];
-      double pij, xij = 0.0;
-      if (A.domain == kLog) {
-        xij = (A.kernel_given ? mij : -mij * inv_reg) + ui + v[j];
-        pij = exp(xij);
-      } else {
-        const double kij = A.kernel_given ? mij : exp(-mij * inv_reg);
-        pij = ui * kij * v[j];
+  const int r0 = (blockIdx.x / A.csplit) * A.rpb, r1 = min(n, r0 + A.rpb);
+  for (int j0 = ((blockIdx.x % A.csplit) * TX + tx) * VEC; j0 < m; j0 += A.csplit * TX * VEC) {
+    double vj[VEC], bj[VEC];
+#pragma unroll
+    for (int c = 0; c < VEC; ++c) {
+      vj[c] = v[j0 + c];
+      bj[c] = kl ? A.b[(int64_t)p * m + j0 + c] : 1.0;
+    }
+    constexpr int Q = 4;
+    for (int i0 = r0 + ty; i0 < r1; i0 += Q * TY) {
+      V x[Q];
+      double ui[Q];
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const int i = min(i0 + q * TY, r1 - 1);
+        x[q] = *reinterpret_cast<const V*>(Mp + (int64_t)i * A.ldm + j0);
+        ui[q] = u[i];
       }
-      if (P) P[(int64_t)i * m + j] = (TM)pij;
-      if (L) L[(int64_t)i * m + j] = (TM)xij;
-      s_cost += mij * pij;
-      s_ent += pij * log(pij + 1e-16);
-      if (A.b) {
-        const double bj = A.b[(int64_t)p * m + j];
-        s_kl += pij * log(pij / (ai * bj) + 1e-16);
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const int i = i0 + q * TY;
+        if (i >= r1) break;
+        V out, lout;
+        const double ai = kl ? A.a[(int64_t)p * n + i] : 1.0;
+#pragma unroll
+        for (int c = 0; c < VEC; ++c) {
+          const double mij = (double)x[q].x[c];
+          double pij, xij = 0.0;
+          if (!SUMS && sizeof(TM) == 4) {
+            if (logd) {
+              pij = exp2_for_f32(fma(mij, s2, (ui[q] + vj[c]) * kLog2e));
+              if (L) xij = (given ? mij : -mij * inv_reg) + ui[q] + vj[c];
+            } else {
+              pij = ui[q] * (given ? mij : exp2_for_f32(mij * s2)) * vj[c];
+            }
+          } else if (logd) {
+            xij = (given ? mij : -mij * inv_reg) + ui[q] + vj[c];
+            pij = exp(xij);
+          } else {
+            const double kij = given ? mij : exp(-mij * inv_reg);
+            pij = ui[q] * kij * vj[c];
+          }
+          out.x[c] = (TM)pij;
+          lout.x[c] = (TM)xij;
+          if (SUMS) {
+            s_cost += mij * pij;
+            if (ent) s_ent += pij * log(pij + 1e-16);
+            if (kl) s_kl += pij * log(pij / (ai * bj[c]) + 1e-16);
+            s_mass += pij;
+          }
+        }
+        if (P) *reinterpret_cast<V*>(P + (int64_t)i * m + j0) = out;
+        if (L) *reinterpret_cast<V*>(L + (int64_t)i * m + j0) = lout;
       }
-      s_mass += pij;
     }
   }
+  if (!SUMS) return;
   __shared__ double red[kPlanSums][kPlanThreads / kWave];
-  double vals[kPlanSums] = {s_cost, s_ent, s_kl, s_mass};
+  const double vals[kPlanSums] = {s_cost, s_ent, s_kl, s_mass};
 #pragma unroll
   for (int q = 0; q < kPlanSums; ++q) {
-    const double w = wave_sum(vals[q]);
+    const double w = wave_sum_dpp_d(vals[q]);
     if ((threadIdx.x & (kWave - 1)) == 0) red[q][threadIdx.x / kWave] = w;
   }
   __syncthreads();
@@ -67,28 +138,69 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs A) {
   }
 }
 
-__global__ void plan_sums_kernel(int nblk, const double* partial, double* sums) {
+// Adds a problem's block partials: 64 strided sums for each of the four, then
+// the sums of a wave in a fixed order.  (One thread over 2048 blocks, a load
+// at a time, took 270 us.)
+__global__ __launch_bounds__(kPlanThreads) void plan_sums_kernel(int nblk, const double* partial,
+                                                                 double* sums) {
   const int p = blockIdx.x;
-  const int q = threadIdx.x;
-  if (q >= kPlanSums) return;
+  const int lane = threadIdx.x & (kWave - 1), q = threadIdx.x / kWave;
+  const double* src = partial + (int64_t)p * nblk * kPlanSums + q;
   double t = 0;
-  for (int b = 0; b < nblk; ++b) t += partial[((int64_t)p * nblk + b) * kPlanSums + q];
-  sums[(int64_t)p * kPlanSums + q] = t;
+#pragma unroll 4
+  for (int b = lane; b < nblk; b += kWave) t += src[(int64_t)b * kPlanSums];
+  t = wave_sum_dpp_d(t);
+  if (lane == 0) sums[(int64_t)p * kPlanSums + q] = t;
 }
 
-int plan_blocks(int n) { return (n + 7) / 8; }
+// Most blocks of a problem's plan (the partials of its sums).
+int plan_blocks(int n) { return (n + 7) / 8 + 8; }
 
 hipError_t launch_plan(int dtype, PlanArgs a, int B, double* sums, hipStream_t s) {
-  const int nblk = plan_blocks(a.n);
-  a.rpb = 8;
+  const int wide = dtype == 0 ? 4 : 2;
+  auto aligned = [&](const void* q, int64_t stride) {
+    return (uintptr_t)q % 16 == 0 && stride % wide == 0;
+  };
+  const bool vec = a.m % wide == 0 && aligned(a.M, a.ldm) && aligned(a.M, a.bstride) &&
+                   aligned(a.P, a.pstride) && aligned(a.logP, a.pstride);
+  const int v = vec ? wide : 1;
+  a.tx = 3;
+  while (a.tx < 8 && (v << a.tx) < a.m) ++a.tx;
+  const int ty = kPlanThreads >> a.tx;
+  const int chunks = (a.m + (v << a.tx) - 1) / (v << a.tx);
+  // Rows of a block: 16 for each row thread, fewer while that leaves the chip
+  // (256 CUs, 8 blocks each) without work; then the column chunks are split.
+  int rows = 16 * ty;
+  auto blocks = [&](int r) { return (a.n + r - 1) / r; };
+  while (rows > 4 * ty && (int64_t)B * blocks(rows) * chunks < 2048) rows -= 4 * ty;
+  rows = std::max(rows, 8);
+  a.rpb = rows;
+  const int nrow = blocks(rows);
+  a.csplit = std::max(1, std::min(chunks, plan_blocks(a.n) / nrow));
+  const int nblk = nrow * a.csplit;
   dim3 grid(nblk, B);
-  if (dtype == 0)
-    hipLaunchKernelGGL(plan_kernel<float>, grid, dim3(kPlanThreads), 0, s, a);
-  else
-    hipLaunchKernelGGL(plan_kernel<double>, grid, dim3(kPlanThreads), 0, s, a);
+#define POTAMD_PLAN(TM, VEC)                                                              \
+  if (sums)                                                                               \
+    hipLaunchKernelGGL((plan_kernel<TM, VEC, true>), grid, dim3(kPlanThreads), 0, s, a);  \
+  else                                                                                    \
+    hipLaunchKernelGGL((plan_kernel<TM, VEC, false>), grid, dim3(kPlanThreads), 0, s, a);
+  if (dtype == 0) {
+    if (vec) {
+      POTAMD_PLAN(float, 4)
+    } else {
+      POTAMD_PLAN(float, 1)
+    }
+  } else {
+    if (vec) {
+      POTAMD_PLAN(double, 2)
+    } else {
+      POTAMD_PLAN(double, 1)
+    }
+  }
+#undef POTAMD_PLAN
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || !sums) return e;
-  hipLaunchKernelGGL(plan_sums_kernel, dim3(B), dim3(64), 0, s, nblk, a.partial, sums);
+  hipLaunchKernelGGL(plan_sums_kernel, dim3(B), dim3(kPlanThreads), 0, s, nblk, a.partial, sums);
   return hipGetLastError();
 }
 

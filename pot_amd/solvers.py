@@ -121,10 +121,12 @@ def solve(M, a=None, b=None, reg=None, c=None, reg_type="KL", unbalanced=None,
         v = res.v
         niter = max_iter + 1
 
-    P, _, sums = _solve.plan(Mt, u, v, reg, domain=_lib.LOG, a=at.view(1, n),
-                             b=bt.view(1, m))
+    ent = reg_type.lower() == "entropy"
+    P, _, sums = _solve.plan(Mt, u, v, reg, domain=_lib.LOG, a=at.view(1, n), b=bt.view(1, m),
+                             want_sums=_solve.SUM_COST | (_solve.SUM_ENTROPY if ent
+                                                          else _solve.SUM_KL))
     value_linear = float(sums[0, 0])
-    reg_term = float(sums[0, 1] if reg_type.lower() == "entropy" else sums[0, 2])
+    reg_term = float(sums[0, 1] if ent else sums[0, 2])
     value = value_linear + reg * reg_term
     plan = ing.out(P[0])
     log_u, log_v = ing.out(u[0]), ing.out(v[0])

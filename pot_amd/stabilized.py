@@ -119,7 +119,7 @@ def _stabilized_multi(ing, Mt, at, bt, reg, numItermax, tau, stopThr, warmstart,
     logu = alpha[None, :] / reg + torch.log(u)  # (H, n)
     logv = beta[None, :] / reg + torch.log(v)
     _, _, sums = _solve.plan(Mt, logu, logv, reg, domain=_lib.LOG, want_plan=False,
-                             batch=H, bstride=0)
+                             want_sums=_solve.SUM_COST, batch=H, bstride=0)
     out = ing.out(sums[:, 0])
     if not log:
         return out
@@ -149,7 +149,8 @@ def sinkhorn_stabilized(a, b, M, reg, numItermax=1000, tau=1e3, stopThr=1e-9, wa
     logu = alpha / reg + torch.log(u)
     logv = beta / reg + torch.log(v)
     P, _, sums = _solve.plan(Mt, logu.view(1, -1), logv.view(1, -1), reg, domain=_lib.LOG,
-                             want_plan=not _loss_only)
+                             want_plan=not _loss_only,
+                             want_sums=_solve.SUM_COST if _loss_only else 0)
     out = ing.scalar(float(sums[0, 0])) if _loss_only else ing.out(P[0])
     if log:
         al = alpha + reg * torch.log(u)
@@ -209,7 +210,7 @@ def sinkhorn_epsilon_scaling(a, b, M, reg, numItermax=100, epsilon0=1e4, numInne
     logu = al / regi + torch.log(u)
     logv = be / regi + torch.log(v)
     P, _, _ = _solve.plan(Mt, logu.view(1, -1), logv.view(1, -1), regi, domain=_lib.LOG,
-                          want_sums=False)
+                          want_sums=0)
     G = ing.out(P[0])
     if log:
         logd = {"err": [ing.scalar(e) for e in errs], "alpha": ing.out(alpha),
