@@ -79,7 +79,25 @@ struct ResidentArgs {
   int row_slot, col_slot;
   int64_t err_slot, col_base, err_base;
   Ctrl* ctrl;            // counter != 0: abandoned
+  // stabilised: u_in / v_in hold alpha / beta
+  int stab, period;
+  double reg, inv_reg, tau, u_start, v_start;
+  double* alpha_out;
+  double* beta_out;
 };
+
+// Threads are 4 W x 16, with ER x EC elements each.
+struct ResidentTile {
+  int W, ER, EC;
+  int rows() const { return 4 * W * ER; }
+  int cols() const { return 16 * EC; }
+};
+hipError_t resident_launch_f32(const ResidentTile& t, const ResidentArgs& a, int grid, size_t lds,
+                               hipStream_t s, int* per_cu);
+hipError_t resident_launch_f64(const ResidentTile& t, const ResidentArgs& a, int grid, size_t lds,
+                               hipStream_t s, int* per_cu);
+hipError_t resident_launch_stab(int f32, const ResidentTile& t, const ResidentArgs& a, int grid,
+                                size_t lds, hipStream_t s, int* per_cu);
 
 bool resident_fits(int dtype, int B, int n, int m);
 size_t resident_workspace(int dtype, int B, int n, int m);

@@ -416,6 +416,7 @@ struct StabLayout {
   double* blk;
   double* rowerr;
   StabCtrl* sc;
+  char* words;  // exchange slots of the register-resident solve
   size_t bytes;
 };
 
@@ -431,8 +432,22 @@ StabLayout carve_stab(void* ws, int dtype, int n, int m, int H) {
   L.blk = c.take<double>(std::max(6 * 1024, (m + 255) / 256 + 8));
   L.rowerr = c.take<double>(n);
   L.sc = c.take<StabCtrl>(1);
+  L.words = c.take<char>(H == 1 ? resident_workspace(POTAMD_F64, 1, n, m) : 0);
   L.bytes = c.off;
   return L;
+}
+
+template <typename TM>
+hipError_t launch_marg(const TM* K, int n, int m, const double* u, const double* v,
+                       const double* a, const double* b, const StabLayout& L, double* marg_sq,
+                       hipStream_t s) {
+  const int G = (n + kColRows - 1) / kColRows;
+  hipLaunchKernelGGL((stab_col_partial<TM>), dim3((m + 255) / 256, G), dim3(256), 0, s, K, n, m,
+                     u, L.part, (const StabCtrl*)nullptr);
+  hipLaunchKernelGGL((stab_row_marg<TM>), dim3(n), dim3(256), 0, s, K, n, m, u, v, a, L.rowerr);
+  hipLaunchKernelGGL(stab_marg_final, dim3(1), dim3(256), 0, s, L.part, G, m, b, v, L.rowerr, n,
+                     marg_sq);
+  return hipGetLastError();
 }
 
 // H histograms (u: H x n, v and b: H x m, histogram-major); `multi` gives
@@ -451,6 +466,54 @@ int run_stabilized(const TM* M, int64_t ldm, int n, int m, int H, bool multi, do
   const dim3 g1s((unsigned)((std::max(n, m) + 255) / 256));
   const int kblocks = (int)std::min<int64_t>(4096, ((int64_t)n * m + 255) / 256);
   const int cblocks = (int)std::min<int64_t>(1024, (nm + 255) / 256);
+  // One histogram whose cost fits the register files: one launch (the ten
+  // launches of an iteration below took 100 us at 1000 x 900 and at 120 x 100;
+  // 13 us and 3 us here, absorbing in most).  What it abandons (a scaling not
+  // finite) is done again here.
+  if (!multi && resident_fits(POTAMD_F64, 1, n, m)) {
+    ResidentArgs r;
+    memset(&r, 0, sizeof(r));
+    r.stab = 1;
+    r.M = M;
+    r.ldm = ldm;
+    r.n = n;
+    r.m = m;
+    r.B = 1;
+    r.a = a;
+    r.b = b;
+    r.u_in = r.alpha_out = alpha;
+    r.v_in = r.beta_out = beta;
+    r.u_out = u;
+    r.v_out = v;
+    r.u_start = 1.0 / n;
+    r.v_start = 1.0 / m;
+    r.reg = reg;
+    r.inv_reg = 1.0 / reg;
+    r.tau = tau;
+    r.period = print_period;
+    r.max_iter = max_iter;
+    r.stop_thr = stop_thr;
+    r.err_hist = err_hist;
+    r.err_cap = err_cap;
+    r.words = reinterpret_cast<unsigned long long*>(L.words);
+    r.ctrl = &L.sc->c;
+    Ctrl got;
+    const int done = resident_solve(sizeof(TM) == 4 ? POTAMD_F32 : POTAMD_F64, r, L.up, L.vp,
+                                    static_cast<Ctrl*>(host_ctrl), s, &got);
+    if (done < 0) return POTAMD_EHIP;
+    if (done == 0) {
+      if (marg_sq) {
+        hipLaunchKernelGGL((stab_build_k<TM>), dim3(kblocks), dim3(256), 0, s, M, ldm, n, m, reg,
+                           alpha, beta, K, (const StabCtrl*)nullptr);
+        HIP_TRY(launch_marg<TM>(K, n, m, u, v, a, b, L, marg_sq, s));
+      }
+      info[0] = got.niter;
+      info[1] = got.n_err;
+      info[2] = got.status;
+      info[3] = got.bad_iter;
+      return got.status;
+    }
+  }
   hipLaunchKernelGGL(stab_init, g1, dim3(256), 0, s, L.sc, u, nu, 1.0 / n, v, nv, 1.0 / m);
   hipLaunchKernelGGL((stab_build_k<TM>), dim3(kblocks), dim3(256), 0, s, M, ldm, n, m, reg,
                      alpha, beta, K, (const StabCtrl*)nullptr);
@@ -549,14 +612,8 @@ int run_stabilized(const TM* M, int64_t ldm, int n, int m, int H, bool multi, do
   for (int k = 0; k < kRing; ++k) (void)hipEventDestroy(ev[k]);
   if (rc) return rc;
   if (marg_sq && !multi) {
-    // the stop flag is set by now; rebuild the partials without it
-    hipLaunchKernelGGL((stab_col_partial<TM>), dim3((m + 255) / 256, G), dim3(256), 0, s, K, n,
-                       m, u, L.part, (const StabCtrl*)nullptr);
-    hipLaunchKernelGGL((stab_row_marg<TM>), dim3(n), dim3(256), 0, s, K, n, m, u, v, a,
-                       L.rowerr);
-    hipLaunchKernelGGL(stab_marg_final, dim3(1), dim3(256), 0, s, L.part, G, m, b, v, L.rowerr,
-                       n, marg_sq);
-    HIP_TRY(hipGetLastError());
+    // the stop flag is set by now; the partials are formed without it
+    HIP_TRY(launch_marg<TM>(K, n, m, u, v, a, b, L, marg_sq, s));
   }
   HIP_TRY(hipMemcpyAsync(&local, L.sc, sizeof(StabCtrl), hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));

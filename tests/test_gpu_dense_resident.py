@@ -14,6 +14,8 @@ import torch
 
 import oracle.batch as ob
 import oracle.sinkhorn as osk
+import oracle.stabilized as ostab
+import pot_amd
 from pot_amd import _lib, _solve
 
 pytestmark = pytest.mark.gpu
@@ -151,3 +153,29 @@ def test_numerical_errors_are_the_row_sweeps():
     got = _solve_gpu(M, a, b, 0.05, **kw)
     assert got.status == want.status == _lib.NUMERICAL
     assert got.bad_iter == want.bad_iter and torch.equal(got.u, want.u)
+
+
+@pytest.mark.parametrize("dtype", [F64, F32])
+@pytest.mark.parametrize("n,m,tau,iters", [(64, 64, 1e3, 1), (65, 33, 2.0, 45), (120, 100, 1e3, 80),
+                                           (300, 260, 3.0, 60), (30, 700, 1e3, 41),
+                                           (700, 30, 5.0, 41)])
+def test_stabilized_absorbs_as_the_oracle(n, m, tau, iters, dtype):
+    """Absorption now and then, at every iteration and in the last one, with
+    one block and with rows or columns (or both) in several."""
+    M, a, b = _problem(1, n, m, dtype, n + m)
+    reg = 0.005
+    P, log = ostab.sinkhorn_stabilized(a[0], b[0], M[0].astype(np.float64), reg, numItermax=iters,
+                                       tau=tau, log=True, warn=False)
+    got, lg = pot_amd.sinkhorn(torch.tensor(a[0], device="cuda"), torch.tensor(b[0], device="cuda"),
+                               torch.tensor(M[0], device="cuda"), reg,
+                               method="sinkhorn_stabilized", numItermax=iters, tau=tau, log=True,
+                               warn=False)
+    assert lg["n_iter"] == log["n_iter"] and len(lg["err"]) == len(log["err"])
+    # float64: a few ulp of exponents up to 1 / reg an iteration; float32: K is
+    # stored in float32
+    tol = 1e-10 if dtype == F64 else 1e-5
+    assert np.max(np.abs(got.cpu().numpy() - P)) < tol * P.max()
+    for key in ("alpha", "beta"):
+        assert np.max(np.abs(lg[key].double().cpu().numpy() - log[key])) < tol
+    np.testing.assert_allclose([float(e) for e in lg["err"]], log["err"], rtol=max(tol, 1e-6),
+                               atol=1e-12 if dtype == F64 else 1e-7)
