@@ -31,9 +31,10 @@
 // error ||P^T 1 - b||_2 (from the column sums the next update needs anyway)
 // and takes the stop decision on the device (last-block ticket).
 //
-// Precisions of x . y^T: fp32 MFMA (32x32x2), bf16 MFMA (32x32x16), bf16
-// hi+lo split with three products (compensated), fp8 e4m3 (32x32x16) with a
-// per-point scale applied in the epilogue, and an fp64 vector-ALU pass that
+// Precisions of x . y^T: fp32 as three bf16 parts (their sum is the fp32 value
+// itself) with the six products that count, on bf16 MFMA (32x32x16); bf16;
+// bf16 hi+lo split with three products (compensated); fp8 e4m3 (32x32x16) with
+// a per-point scale applied in the epilogue; and an fp64 vector-ALU pass that
 // serves as the full-size reference.  Exponents, sums and potentials are
 // fp32 / fp64 as described above in every variant.
 #include <math.h>
@@ -48,8 +49,7 @@
 namespace potamd {
 namespace {
 
-constexpr int kRowsPerWG = 128;  // R points per workgroup of the MFMA pass
-constexpr int kStep = 64;        // C points per LDS stage
+constexpr int kStep = 64;        // C points that splits are made of
 constexpr int kPad = 128;        // packed operands are padded to this many points
 constexpr float kFp8Max = 224.f; // largest |q| of a scaled fp8 operand
 
@@ -58,12 +58,13 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
-template <int P> struct Op;
-template <> struct Op<POTAMD_ONLINE_F32> { static constexpr int es = 4; static constexpr bool lo = false; };
-template <> struct Op<POTAMD_ONLINE_BF16> { static constexpr int es = 2; static constexpr bool lo = false; };
-template <> struct Op<POTAMD_ONLINE_BF16X3> { static constexpr int es = 2; static constexpr bool lo = true; };
-template <> struct Op<POTAMD_ONLINE_FP8> { static constexpr int es = 1; static constexpr bool lo = false; };
-template <> struct Op<POTAMD_ONLINE_F64> { static constexpr int es = 4; static constexpr bool lo = false; };
+// Element size and parts (planes) of an operand, C points of an LDS stage.
+template <int P> struct Op { static constexpr int es = 2, parts = 1, stage = 64; };
+template <> struct Op<POTAMD_ONLINE_F32> { static constexpr int es = 2, parts = 3, stage = 32; };
+template <> struct Op<POTAMD_ONLINE_BF16X3> { static constexpr int es = 2, parts = 2, stage = 64; };
+template <> struct Op<POTAMD_ONLINE_FP8> { static constexpr int es = 1, parts = 1, stage = 64; };
+constexpr int kWaves = 4;        // of a workgroup, 32 R points each
+constexpr int kRowsPerWG = 32 * kWaves;
 
 __device__ __forceinline__ unsigned short bf16_rne(float f) {
   unsigned int u = __float_as_uint(f);
@@ -89,6 +90,12 @@ __device__ __forceinline__ u32x2 split4_bf16(double x) {
   return u32x2{q[0] | (q[1] << 16), q[2] | (q[3] << 16)};
 }
 constexpr unsigned kOnes = 0x3F803F80u;  // two bf16 1.0
+
+// x to a multiple of 2^-10 (to fp32 beyond 2^13): the difference of two of
+// them is exact in fp32.
+__device__ __forceinline__ float coarse(double x) {
+  return fabs(x) < 8192.0 ? (float)(rint(x * 1024.0) * 0.0009765625) : (float)x;
+}
 
 // t <- exp2(t) elementwise; returns the sum of the 16 values as a pairwise
 // tree.
@@ -125,8 +132,7 @@ struct PackArgs {
   const double* cscale;
   double reg;
   int scaled;
-  void* pk;
-  void* pk_lo;
+  void* pk;           // planes of rows_pad x D, one after the other
   float* pk_scale;
   double* norms;
 };
@@ -155,27 +161,23 @@ __global__ __launch_bounds__(256) void online_pack_kernel(PackArgs A) {
     if (row < A.rows && e < A.d) x = (float)coord(A.X, (int64_t)row * A.ldx + e, A.x64);
     t[j] = (float)((double)x * sc);
   }
-  if constexpr (P == POTAMD_ONLINE_F32) {
+  if constexpr (P != POTAMD_ONLINE_FP8) {
     if (e0 < A.D) {
-      float* o = static_cast<float*>(A.pk) + (int64_t)row * A.D + e0;
-      *reinterpret_cast<float4*>(o) = make_float4(t[0], t[1], t[2], t[3]);
-    }
-  } else if constexpr (P == POTAMD_ONLINE_BF16 || P == POTAMD_ONLINE_BF16X3) {
-    if (e0 < A.D) {
-      unsigned short hi[4], lo[4];
+      unsigned short* o = static_cast<unsigned short*>(A.pk) + (int64_t)row * A.D + e0;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        hi[j] = bf16_rne(t[j]);
-        lo[j] = bf16_rne(t[j] - bf16_val(hi[j]));
-      }
-      u32x2 wh = {(unsigned)hi[0] | ((unsigned)hi[1] << 16), (unsigned)hi[2] | ((unsigned)hi[3] << 16)};
-      *reinterpret_cast<u32x2*>(static_cast<unsigned short*>(A.pk) + (int64_t)row * A.D + e0) = wh;
-      if constexpr (P == POTAMD_ONLINE_BF16X3) {
-        u32x2 wl = {(unsigned)lo[0] | ((unsigned)lo[1] << 16), (unsigned)lo[2] | ((unsigned)lo[3] << 16)};
-        *reinterpret_cast<u32x2*>(static_cast<unsigned short*>(A.pk_lo) + (int64_t)row * A.D + e0) = wl;
+      for (int q = 0; q < Op<P>::parts; ++q) {
+        unsigned short part[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          part[j] = bf16_rne(t[j]);
+          t[j] -= bf16_val(part[j]);  // exact; nothing is left after the third
+        }
+        *reinterpret_cast<u32x2*>(o + (int64_t)q * A.rows_pad * A.D) =
+            u32x2{(unsigned)part[0] | ((unsigned)part[1] << 16),
+                  (unsigned)part[2] | ((unsigned)part[3] << 16)};
       }
     }
-  } else if constexpr (P == POTAMD_ONLINE_FP8) {
+  } else {
     float am = fmaxf(fmaxf(fabsf(t[0]), fabsf(t[1])), fmaxf(fabsf(t[2]), fabsf(t[3])));
     am = wave_max(am);
     const float sig = am > 0.f ? am / kFp8Max : 1.f;
@@ -193,10 +195,8 @@ __global__ __launch_bounds__(256) void online_pack_kernel(PackArgs A) {
 // MFMA pass.
 struct PassArgs {
   const void* r_pk;
-  const void* r_lo;
   const float* r_sc;
   const void* c_pk;
-  const void* c_lo;
   const float* c_sc;
   const double* c_pot;   // C potential, base 2 (LSE mode)
   const double* c_norm;  // |c|^2, fp64
@@ -207,7 +207,7 @@ struct PassArgs {
   double reg;
   double* part;   // [splits][nr_pad]
   int* part_idx;  // max mode: arg max
-  int nr_pad;
+  int nr_pad, nc_pad;
   const Ctrl* ctrl;
 };
 
@@ -215,12 +215,7 @@ enum PassMode : int { kModeLse = 0, kModeMax = 1 };
 
 template <int P>
 __device__ __forceinline__ void mma_chunk(f32x16& acc, u32x4 a, u32x4 b) {
-  if constexpr (P == POTAMD_ONLINE_F32) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a[j]), __uint_as_float(b[j]),
-                                                 acc, 0, 0, 0);
-  } else if constexpr (P == POTAMD_ONLINE_FP8) {
+  if constexpr (P == POTAMD_ONLINE_FP8) {
     const long a0 = (long)(((unsigned long)a[1] << 32) | a[0]);
     const long a1 = (long)(((unsigned long)a[3] << 32) | a[2]);
     const long b0 = (long)(((unsigned long)b[1] << 32) | b[0]);
@@ -233,21 +228,33 @@ __device__ __forceinline__ void mma_chunk(f32x16& acc, u32x4 a, u32x4 b) {
   }
 }
 
-// bf16x3 at d = 64 needs a few registers more than three waves per SIMD
-// allow; the pass is latency-bound there, so three waves are asked for.
+// Three waves a SIMD are asked for where the register need is close to that:
+// with two, the matrix core waits for the other wave's exponentials.
+//
+// fp32: x = h + m + l in bf16 parts (|m| <= 2^-9 |x|, |l| <= 2^-18 |x|), and
+// h.l + l.h + m.m + h.m + m.h in one accumulator, h.h in another; what is left
+// out (m.l, l.m, l.l) is below 2^-26 of a product.  At 16 times the rate of
+// the fp32 matrix instructions, 6 products take 3/8 of their time, and the
+// error of x . y is a third (rms 6e-8 of its mean size at d = 64, against
+// 1.8e-7: 9 roundings of full size for 32).  16384^2 points, d = 64: 201 us a
+// pass, 313 before; matrix cores 46% busy, VALU 37%.  d <= 16 takes one K step
+// of 16 instead of two: 5000 x 4000 points in 3-D, 14.4 us a pass, 22 before.
 template <int P, int D, int MODE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
-    (P == POTAMD_ONLINE_BF16X3 && D == 64 && MODE == kModeLse) ? 3 : 1)))
+__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(
+    ((P == POTAMD_ONLINE_BF16X3 && D == 64) || (P == POTAMD_ONLINE_F32 && D <= 64)) && MODE == kModeLse
+        ? 3 : 1)))
 void online_pass_kernel(PassArgs A) {
   if (A.ctrl && A.ctrl->done) return;
   constexpr int es = Op<P>::es;
-  constexpr bool LO = Op<P>::lo;
+  constexpr int PARTS = Op<P>::parts;
+  constexpr int T = 64 * kWaves;
+  constexpr int SS = Op<P>::stage;
   constexpr bool FP8 = P == POTAMD_ONLINE_FP8;
   constexpr int ROWB = D * es + 16;           // LDS bytes per C point (padded)
-  constexpr int TILE = kStep * ROWB;
+  constexpr int TILE = SS * ROWB;
   constexpr int CPR = D * es / 16;            // 16-byte chunks per point
-  constexpr int NCHUNK = kStep * CPR;         // chunks per stage
-  constexpr int NPT = (NCHUNK + 255) / 256;   // chunks per thread
+  constexpr int NCHUNK = SS * CPR;         // chunks per stage
+  constexpr int NPT = (NCHUNK + T - 1) / T;   // chunks per thread and part
   constexpr int NB = D * es / 32;             // 16-byte chunks per lane (half a point)
   // bf16 operands: the potential term enters the accumulator through one
   // more bf16 MFMA (K slots [P1..P4, 1, 1, 1, 1] x [1, 1, 1, 1, -Q1..-Q4],
@@ -255,11 +262,10 @@ void online_pass_kernel(PassArgs A) {
   // parts), issued after the dot product.
   constexpr bool KS = MODE == kModeLse && (P == POTAMD_ONLINE_BF16 || P == POTAMD_ONLINE_BF16X3);
 
-  __shared__ __attribute__((aligned(16))) char sm_t[2][TILE];
-  __shared__ __attribute__((aligned(16))) char sm_lo[LO ? 2 : 1][LO ? TILE : 16];
-  __shared__ double sm_v[2][kStep];
-  __shared__ float sm_sc[2][kStep];
-  __shared__ u32x2 sm_kp[KS ? 2 : 1][KS ? kStep : 1];
+  __shared__ __attribute__((aligned(16))) char sm_t[2][PARTS][TILE];
+  __shared__ __attribute__((aligned(16))) double sm_v[2][SS];  // fp32: (high, low) floats
+  __shared__ float sm_sc[2][SS];
+  __shared__ u32x2 sm_kp[KS ? 2 : 1][KS ? SS : 1];
 
   const int tid = threadIdx.x;
   const int wave = tid >> 6;
@@ -268,23 +274,19 @@ void online_pass_kernel(PassArgs A) {
   const int l32 = lane & 31;
   const int r = blockIdx.x * kRowsPerWG + wave * 32 + l32;
   const int split = blockIdx.y;
-  const int nsteps = (A.nc + kStep - 1) / kStep;
-  const int step0 = split * A.steps_per_split;
-  const int step1 = min(step0 + A.steps_per_split, nsteps);
+  const int nsteps = (A.nc + SS - 1) / SS;
+  const int step0 = split * A.steps_per_split * (kStep / SS);
+  const int step1 = min(step0 + A.steps_per_split * (kStep / SS), nsteps);
   const double s2 = MODE == kModeLse ? s2_of(A.cscale, A.reg) : 0.0;
 
   // R operand: half a point per lane, for the whole pass.
-  u32x4 rb[NB];
-  u32x4 rl[LO ? NB : 1];
-  {
-    const char* rp = static_cast<const char*>(A.r_pk) + ((int64_t)r * D + h * (D / 2)) * es;
+  u32x4 rb[PARTS][NB];
 #pragma unroll
-    for (int i = 0; i < NB; ++i) rb[i] = *reinterpret_cast<const u32x4*>(rp + 16 * i);
-    if constexpr (LO) {
-      const char* lp = static_cast<const char*>(A.r_lo) + ((int64_t)r * D + h * (D / 2)) * es;
+  for (int q = 0; q < PARTS; ++q) {
+    const char* rp = static_cast<const char*>(A.r_pk) +
+                     (((int64_t)q * A.nr_pad + r) * D + h * (D / 2)) * es;
 #pragma unroll
-      for (int i = 0; i < NB; ++i) rl[i] = *reinterpret_cast<const u32x4*>(lp + 16 * i);
-    }
+    for (int i = 0; i < NB; ++i) rb[q][i] = *reinterpret_cast<const u32x4*>(rp + 16 * i);
   }
   const float r_sig = FP8 ? A.r_sc[r] : 1.f;
 
@@ -293,7 +295,7 @@ void online_pass_kernel(PassArgs A) {
   if (MODE == kModeLse && A.r_shift) {
     const double s0 = A.r_shift[r];
     if (__builtin_isfinite(s0)) {
-      cl = s0;
+      cl = PARTS == 3 ? (double)coarse(s0) : s0;
       fresh = false;
     }
   }
@@ -310,30 +312,23 @@ void online_pass_kernel(PassArgs A) {
   int best_c = 0;
 
   // Stage loader: C points [step*64, step*64 + 64) into registers.
-  u32x4 st[NPT];
-  u32x4 stl[LO ? NPT : 1];
+  u32x4 st[PARTS][NPT];
   double st_v = 0.0;
   float st_sc = 1.f;
   u32x2 st_kp = {0u, 0u};
   auto load = [&](int step) {
-    const int64_t c0 = (int64_t)step * kStep;
-    const char* cp = static_cast<const char*>(A.c_pk) + c0 * D * es;
+    const int64_t c0 = (int64_t)step * SS;
 #pragma unroll
-    for (int i = 0; i < NPT; ++i) {
-      const int q = tid + 256 * i;
-      if (NCHUNK % 256 == 0 || q < NCHUNK)
-        st[i] = *reinterpret_cast<const u32x4*>(cp + (int64_t)(q / CPR) * D * es + (q % CPR) * 16);
-    }
-    if constexpr (LO) {
-      const char* lp = static_cast<const char*>(A.c_lo) + c0 * D * es;
+    for (int p = 0; p < PARTS; ++p) {
+      const char* cp = static_cast<const char*>(A.c_pk) + ((int64_t)p * A.nc_pad + c0) * D * es;
 #pragma unroll
       for (int i = 0; i < NPT; ++i) {
-        const int q = tid + 256 * i;
-        if (NCHUNK % 256 == 0 || q < NCHUNK)
-          stl[i] = *reinterpret_cast<const u32x4*>(lp + (int64_t)(q / CPR) * D * es + (q % CPR) * 16);
+        const int q = tid + T * i;
+        if (NCHUNK % T == 0 || q < NCHUNK)
+          st[p][i] = *reinterpret_cast<const u32x4*>(cp + (int64_t)(q / CPR) * D * es + (q % CPR) * 16);
       }
     }
-    if (tid < kStep) {
+    if (tid < SS) {
       const int64_t c = c0 + tid;
       if (c < A.nc) {
         st_v = MODE == kModeLse ? A.c_pot[c] - s2 * A.c_norm[c] : A.c_norm[c];
@@ -342,25 +337,31 @@ void online_pass_kernel(PassArgs A) {
       }
       if constexpr (FP8) st_sc = A.c_sc[c];
       if constexpr (KS) st_kp = split4_bf16(st_v);
+      if constexpr (PARTS == 3 && MODE == kModeLse) {
+        const float hi = coarse(st_v);
+        const float lo = st_v > -__builtin_inf() ? (float)(st_v - (double)hi) : 0.f;
+        st_v = __builtin_bit_cast(double, u32x2{__float_as_uint(hi), __float_as_uint(lo)});
+      }
     }
   };
   auto store = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < NPT; ++i) {
-      const int q = tid + 256 * i;
-      if (NCHUNK % 256 == 0 || q < NCHUNK)
-        *reinterpret_cast<u32x4*>(&sm_t[buf][(q / CPR) * ROWB + (q % CPR) * 16]) = st[i];
-    }
-    if constexpr (LO) {
+    for (int p = 0; p < PARTS; ++p)
 #pragma unroll
       for (int i = 0; i < NPT; ++i) {
-        const int q = tid + 256 * i;
-        if (NCHUNK % 256 == 0 || q < NCHUNK)
-          *reinterpret_cast<u32x4*>(&sm_lo[buf][(q / CPR) * ROWB + (q % CPR) * 16]) = stl[i];
+        const int q = tid + T * i;
+        if (NCHUNK % T == 0 || q < NCHUNK)
+          *reinterpret_cast<u32x4*>(&sm_t[buf][p][(q / CPR) * ROWB + (q % CPR) * 16]) = st[p][i];
       }
-    }
-    if (tid < kStep) {
-      sm_v[buf][tid] = st_v;
+    if (tid < SS) {
+      if constexpr (PARTS == 3 && MODE == kModeLse) {
+        // all high parts, then all low ones
+        const u32x2 w = __builtin_bit_cast(u32x2, st_v);
+        reinterpret_cast<unsigned*>(sm_v[buf])[tid] = w[0];
+        reinterpret_cast<unsigned*>(sm_v[buf])[SS + tid] = w[1];
+      } else {
+        sm_v[buf][tid] = st_v;
+      }
       if constexpr (FP8) sm_sc[buf][tid] = st_sc;
       if constexpr (KS) sm_kp[buf][tid] = st_kp;
     }
@@ -372,26 +373,57 @@ void online_pass_kernel(PassArgs A) {
   auto tile = [&](int buf, int sb, double shift) -> f32x16 {
     f32x16 acc;
     const double* vrow = &sm_v[buf][sb * 32 + 4 * h];
-    if constexpr (MODE == kModeLse && !FP8 && !KS) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
+    for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+    const int off = (sb * 32 + l32) * ROWB + h * (D / 2) * es;
+    auto part = [&](int p, int i) {
+      return *reinterpret_cast<const u32x4*>(&sm_t[buf][p][off + 16 * i]);
+    };
+    if constexpr (PARTS == 3) {
+      // The small products, smallest before larger, in their own accumulator:
+      // the matrix core cuts an accumulator off (towards -inf) where it is far
+      // below the products it meets, a bias of 5e-9 of x . y (1e-10 this way;
+      // rms 6e-8, the fp32 instructions 1.8e-7).
+      const float* vh = reinterpret_cast<const float*>(sm_v[buf]) + sb * 32 + 4 * h;
+      f32x16 low = acc;
+      if constexpr (MODE == kModeLse) {
 #pragma unroll
-        for (int rr = 0; rr < 4; ++rr) acc[4 * q + rr] = (float)(vrow[8 * q + rr] - shift);
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int rr = 0; rr < 4; ++rr) low[4 * q + rr] = vh[SS + 8 * q + rr];
+      }
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        const u32x4 ah = part(0, i), am = part(1, i), al = part(2, i);
+        mma_chunk<P>(low, al, rb[0][i]);
+        mma_chunk<P>(acc, ah, rb[0][i]);
+        mma_chunk<P>(low, ah, rb[2][i]);
+        mma_chunk<P>(low, am, rb[1][i]);
+        mma_chunk<P>(low, am, rb[0][i]);
+        mma_chunk<P>(low, ah, rb[1][i]);
+      }
+      if constexpr (MODE == kModeLse) {
+        // The potential term: its high part less the shift is exact, its low
+        // part went through the small products (all of it through the matrix
+        // core's K slots left a bias of 8e-8 in the cost <P, M>).
+        const float cf = (float)shift;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int rr = 0; rr < 4; ++rr) acc[4 * q + rr] += vh[8 * q + rr] - cf;
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[i] += low[i];
     } else {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[i] = 0.f;
-    }
-    const char* trow = &sm_t[buf][(sb * 32 + l32) * ROWB + h * (D / 2) * es];
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const u32x4 a = *reinterpret_cast<const u32x4*>(trow + 16 * i);
-      if constexpr (LO) {
-        const char* lrow = &sm_lo[buf][(sb * 32 + l32) * ROWB + h * (D / 2) * es];
-        const u32x4 al = *reinterpret_cast<const u32x4*>(lrow + 16 * i);
-        mma_chunk<P>(acc, a, rl[i]);
-        mma_chunk<P>(acc, al, rb[i]);
+      for (int i = 0; i < NB; ++i) {
+        const u32x4 a = part(0, i);
+        if constexpr (PARTS == 2) {
+          mma_chunk<P>(acc, a, rb[1][i]);
+          mma_chunk<P>(acc, part(1, i), rb[0][i]);
+        }
+        mma_chunk<P>(acc, a, rb[0][i]);
       }
-      mma_chunk<P>(acc, a, rb[i]);
     }
     if constexpr (KS) {
       // Output value i of lane (r, h) is C point 8(i/4) + 4h + i%4 of the
@@ -426,7 +458,7 @@ void online_pass_kernel(PassArgs A) {
     const bool more = step + 1 < step1;
     if (more) load(step + 1);
 #pragma unroll
-    for (int sb = 0; sb < 2; ++sb) {
+    for (int sb = 0; sb < SS / 32; ++sb) {
       f32x16 t = tile(buf, sb, cl);
       if constexpr (MODE == kModeLse) {
         // exp2 in place (no extra registers), then a depth-4 tree sum, so
@@ -439,6 +471,8 @@ void online_pass_kernel(PassArgs A) {
         // and the lane re-centred.
         const bool suspect = fresh || !(ts <= 0x1p20f) || (ts < 0x1p-40f && ssum < 0x1p-40);
         if (__ballot(suspect)) {
+          // (read again: kept operands would cost the common way its registers)
+          asm volatile("" ::: "memory");
           t = tile(buf, sb, cl);
           float tmax = t[0];
 #pragma unroll
@@ -449,11 +483,13 @@ void online_pass_kernel(PassArgs A) {
             if (need) {
               double delta = tmax;
               if (!fresh && ssum > 0.0) delta = fmax(delta, log2(ssum));
-              ssum *= exp2(-delta);
-              cl += delta;
+              const double from = cl;
+              cl = PARTS == 3 ? (double)coarse(cl + delta) : cl + delta;
+              if (!fresh) ssum *= exp2(from - cl);
               fresh = false;
               if constexpr (KS) rkq = shift_slots();
             }
+            asm volatile("" ::: "memory");
             t = tile(buf, sb, cl);
             ts = exp2_tree_sum(t);
           }
@@ -461,7 +497,7 @@ void online_pass_kernel(PassArgs A) {
         ssum += (double)ts;
       } else {
         const double* vrow = &sm_v[buf][sb * 32 + 4 * h];
-        const int cb = step * kStep + sb * 32 + 4 * h;
+        const int cb = step * SS + sb * 32 + 4 * h;
 #pragma unroll
         for (int q = 0; q < 4; ++q)
 #pragma unroll
@@ -951,9 +987,14 @@ __global__ void online_fill_kernel(int64_t count, double val, double* y) {
 
 int round_up(int x, int k) { return (x + k - 1) / k * k; }
 
+// Coordinates are padded to what the matrix instructions of a pass take: 16
+// (bf16 parts, small d), else 32s.
 int padded_dim(int prec, int d) {
-  return prec == POTAMD_ONLINE_F64 ? d : round_up(d, 32);
+  if (prec == POTAMD_ONLINE_F64) return d;
+  return d <= 16 && prec != POTAMD_ONLINE_FP8 ? 16 : round_up(d, 32);
 }
+
+
 
 bool supported(int prec, int d) {
   if (prec < POTAMD_ONLINE_F32 || prec > POTAMD_ONLINE_F64) return false;
@@ -964,8 +1005,6 @@ bool supported(int prec, int d) {
 struct OnlineLayout {
   char* pkX;
   char* pkY;
-  char* loX;
-  char* loY;
   float* scX;
   float* scY;
   double* xn;
@@ -987,7 +1026,7 @@ struct OnlineLayout {
 
 int max_splits(int n, int m) {
   // Splits of the C side for a pass: about 2048 workgroups, at least 4 stages each.
-  const int wgs = round_up(n, kPad) / kRowsPerWG;
+  const int wgs = (n + kRowsPerWG - 1) / kRowsPerWG;
   const int steps = (m + kStep - 1) / kStep;
   int s = (2048 + wgs - 1) / wgs;
   s = std::min(s, std::max(1, steps / 4));
@@ -998,16 +1037,13 @@ OnlineLayout carve_online(void* ws, int prec, int n, int m, int d) {
   Carver c(ws);
   OnlineLayout L;
   memset(&L, 0, sizeof(L));
-  // Operand rows hold the widest format (fp32, also used by the max pass).
+  // Operand rows hold the widest format (three bf16 parts, also used by the
+  // max pass).
   const int Dm = round_up(d, 32);
-  const size_t row_bytes = Dm <= 128 ? (size_t)Dm * 4 : 0;
-  const int D = padded_dim(prec, d);
+  const size_t row_bytes = Dm <= 128 ? (size_t)Dm * 6 : 0;
   const int np = round_up(n, kPad), mp = round_up(m, kPad);
   L.pkX = c.take<char>((size_t)np * row_bytes);
   L.pkY = c.take<char>((size_t)mp * row_bytes);
-  const bool lo = prec == POTAMD_ONLINE_BF16X3;
-  L.loX = c.take<char>(lo ? (size_t)np * D * 2 : 0);
-  L.loY = c.take<char>(lo ? (size_t)mp * D * 2 : 0);
   L.scX = c.take<float>(np);
   L.scY = c.take<float>(mp);
   L.xn = c.take<double>(np);
@@ -1050,12 +1086,17 @@ hipError_t launch_pack(int prec, const PackArgs& a, hipStream_t s) {
 
 template <int P, int MODE>
 hipError_t launch_pass_d(int D, const PassArgs& a, int S, hipStream_t s) {
-  dim3 grid(a.nr_pad / kRowsPerWG, S);
+  constexpr int T = 64 * kWaves;
+  dim3 grid((a.nr + kRowsPerWG - 1) / kRowsPerWG, S);
   switch (D) {
-    case 32: hipLaunchKernelGGL((online_pass_kernel<P, 32, MODE>), grid, dim3(256), 0, s, a); break;
-    case 64: hipLaunchKernelGGL((online_pass_kernel<P, 64, MODE>), grid, dim3(256), 0, s, a); break;
-    case 96: hipLaunchKernelGGL((online_pass_kernel<P, 96, MODE>), grid, dim3(256), 0, s, a); break;
-    default: hipLaunchKernelGGL((online_pass_kernel<P, 128, MODE>), grid, dim3(256), 0, s, a); break;
+    case 16:
+      if constexpr (P != POTAMD_ONLINE_FP8)
+        hipLaunchKernelGGL((online_pass_kernel<P, 16, MODE>), grid, dim3(T), 0, s, a);
+      break;
+    case 32: hipLaunchKernelGGL((online_pass_kernel<P, 32, MODE>), grid, dim3(T), 0, s, a); break;
+    case 64: hipLaunchKernelGGL((online_pass_kernel<P, 64, MODE>), grid, dim3(T), 0, s, a); break;
+    case 96: hipLaunchKernelGGL((online_pass_kernel<P, 96, MODE>), grid, dim3(T), 0, s, a); break;
+    default: hipLaunchKernelGGL((online_pass_kernel<P, 128, MODE>), grid, dim3(T), 0, s, a); break;
   }
   return hipGetLastError();
 }
@@ -1075,7 +1116,6 @@ struct Side {
   int64_t ld;
   int count, pad;
   char* pk;
-  char* lo;
   float* sc;
   double* norm;
   double* shift;
@@ -1112,10 +1152,8 @@ hipError_t half_step(int prec, int D, int d, const Side& R, const Side& C, const
   } else {
     PassArgs pa;
     pa.r_pk = R.pk;
-    pa.r_lo = R.lo;
     pa.r_sc = R.sc;
     pa.c_pk = C.pk;
-    pa.c_lo = C.lo;
     pa.c_sc = C.sc;
     pa.c_pot = c_pot;
     pa.c_norm = C.norm;
@@ -1128,6 +1166,7 @@ hipError_t half_step(int prec, int D, int d, const Side& R, const Side& C, const
     pa.part = L.part;
     pa.part_idx = nullptr;
     pa.nr_pad = R.pad;
+    pa.nc_pad = C.pad;
     pa.ctrl = L.ctrl;
     hipError_t e = launch_pass(prec, D, pa, Seff, s);
     if (e != hipSuccess) return e;
@@ -1201,8 +1240,8 @@ extern "C" int potamd_sinkhorn_online(int precision, int dtype, const void* X, i
   HIP_TRY(fill(np, nan, L.shX, s));
   HIP_TRY(fill(mp, nan, L.shY, s));
 
-  Side SX{X, x64, ldx, n, np, L.pkX, L.loX, L.scX, L.xn, L.shX, a, L.loga2};
-  Side SY{Y, x64, ldy, m, mp, L.pkY, L.loY, L.scY, L.yn, L.shY, b, L.logb2};
+  Side SX{X, x64, ldx, n, np, L.pkX, L.scX, L.xn, L.shX, a, L.loga2};
+  Side SY{Y, x64, ldy, m, mp, L.pkY, L.scY, L.yn, L.shY, b, L.logb2};
 
   PackArgs pk;
   memset(&pk, 0, sizeof(pk));
@@ -1218,7 +1257,6 @@ extern "C" int potamd_sinkhorn_online(int precision, int dtype, const void* X, i
     pk.rows_pad = S.pad;
     pk.scaled = scaled;
     pk.pk = S.pk;
-    pk.pk_lo = S.lo;
     pk.pk_scale = S.sc;
     pk.norms = S.norm;
     return launch_pack(p, pk, s);
@@ -1228,12 +1266,12 @@ extern "C" int potamd_sinkhorn_online(int precision, int dtype, const void* X, i
   if (cost_scale > 0.0) {
     HIP_TRY(fill(1, cost_scale, L.cscale, s));
   } else {
-    const int Dm = round_up(d, 32);
+    const int Dm = padded_dim(POTAMD_ONLINE_F32, d);
     if (Dm > 128) return POTAMD_EUNSUPPORTED;
     pk.D = Dm;
     {
       pk.X = X; pk.ldx = ldx; pk.rows = n; pk.d = d; pk.D = Dm; pk.rows_pad = np; pk.scaled = 0;
-      pk.pk = L.pkX; pk.pk_lo = nullptr; pk.pk_scale = L.scX; pk.norms = L.xn;
+      pk.pk = L.pkX; pk.pk_scale = L.scX; pk.norms = L.xn;
       HIP_TRY(launch_pack(POTAMD_ONLINE_F32, pk, s));
       pk.X = Y; pk.ldx = ldy; pk.rows = m; pk.rows_pad = mp;
       pk.pk = L.pkY; pk.pk_scale = L.scY; pk.norms = L.yn;
@@ -1256,6 +1294,7 @@ extern "C" int potamd_sinkhorn_online(int precision, int dtype, const void* X, i
     pa.part = L.part;
     pa.part_idx = L.pidx;
     pa.nr_pad = np;
+    pa.nc_pad = mp;
     pa.ctrl = nullptr;
     HIP_TRY((launch_pass_d<POTAMD_ONLINE_F32, kModeMax>(Dm, pa, Seff, s)));
     MaxReduceArgs mr;
@@ -1376,7 +1415,7 @@ extern "C" int potamd_sinkhorn_online(int precision, int dtype, const void* X, i
       }
     }
   }
-  for (int k = 0; k < kRing; ++k) hipEventDestroy(ev[k]);
+  for (int k = 0; k < kRing; ++k) (void)hipEventDestroy(ev[k]);
   if (rc) return rc;
   double cs_host = 0.0;
   HIP_TRY(hipMemcpyAsync(&local, L.ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, s));
