@@ -26,10 +26,10 @@
 //    with nothing accumulated yet, which keeps the sum exact at the cost of
 //    a rare extra tile and no per-element maximum;
 //  * partial sums are combined in fp64 (16 fp32 terms per tile each).
-// The merge kernel combines the split partials in fp64, writes the new
+// The last split of a block of R points combines the partials in fp64, writes the new
 // potential, and on the column update computes the reference's marginal
 // error ||P^T 1 - b||_2 (from the column sums the next update needs anyway)
-// and takes the stop decision on the device (last-block ticket).
+// and the stop decision is a one-workgroup kernel after a checking pass.
 //
 // Precisions of x . y^T: fp32 as three bf16 parts (their sum is the fp32 value
 // itself) with the six products that count, on bf16 MFMA (32x32x16); bf16;
@@ -58,11 +58,16 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
-// Element size and parts (planes) of an operand, C points of an LDS stage.
-template <int P> struct Op { static constexpr int es = 2, parts = 1, stage = 64; };
-template <> struct Op<POTAMD_ONLINE_F32> { static constexpr int es = 2, parts = 3, stage = 32; };
-template <> struct Op<POTAMD_ONLINE_BF16X3> { static constexpr int es = 2, parts = 2, stage = 64; };
-template <> struct Op<POTAMD_ONLINE_FP8> { static constexpr int es = 1, parts = 1, stage = 64; };
+// Element size and parts (planes) of an operand.
+template <int P> struct Op { static constexpr int es = 2, parts = 1; };
+template <> struct Op<POTAMD_ONLINE_F32> { static constexpr int es = 2, parts = 3; };
+template <> struct Op<POTAMD_ONLINE_BF16X3> { static constexpr int es = 2, parts = 2; };
+template <> struct Op<POTAMD_ONLINE_FP8> { static constexpr int es = 1, parts = 1; };
+// C points of an LDS stage: enough tiles a stage to cover the next one's loads
+// where d is small, three workgroups a CU where the three fp32 planes are wide.
+constexpr int stage_points(int P, int D) {
+  return D <= 16 ? 128 : P == POTAMD_ONLINE_F32 && D > 32 ? 32 : 64;
+}
 constexpr int kWaves = 4;        // of a workgroup, 32 R points each
 constexpr int kRowsPerWG = 32 * kWaves;
 
@@ -192,6 +197,56 @@ __global__ __launch_bounds__(256) void online_pack_kernel(PackArgs A) {
 }
 
 // ---------------------------------------------------------------------------
+// Merge of the split partials into the new potential of the R side.
+struct OnlineMergeArgs {
+  const double* part;
+  int S, nr, nr_pad;
+  const double* w;       // weights of the R side
+  const double* logw2;   // log2 of the weights
+  const double* norm;    // |r|^2
+  const double* pot_cur; // current potential of the R side (error only)
+  double* pot_new;
+  double* shift;
+  const double* cscale;
+  double reg;
+  int check, decide, iter, max_iter;
+  int l1;         // error: 1 = sum |marginal - w| (empirical_sinkhorn), 0 = 2-norm
+  int inclusive;  // stop: 1 = err <= stop_thr (empirical_sinkhorn), 0 = err < stop_thr
+  double stop_thr;
+  double* err_hist;
+  int err_cap;
+  double* errpart;
+  Ctrl* ctrl;
+};
+
+// New potential and shift of R point r from its S split partials, read by
+// `get`; returns its error term on a check.
+template <typename Get>
+__device__ __forceinline__ double merge_row(const OnlineMergeArgs& A, int r, int S, Get get) {
+  double mx = -__builtin_inf();
+#pragma unroll 8
+  for (int s = 0; s < S; ++s) mx = fmax(mx, get(s));
+  double I = -__builtin_inf();
+  if (mx > -__builtin_inf()) {
+    double acc = 0.0;
+#pragma unroll 8
+    for (int s = 0; s < S; ++s) acc += exp2(get(s) - mx);
+    I = mx + log2(acc);
+  }
+  const double s2 = s2_of(A.cscale, A.reg);
+  const double L2 = I - s2 * A.norm[r];
+  const double wr = A.w[r];
+  double e2 = 0.0;
+  if (A.check) {
+    const double cs = exp2(A.pot_cur[r] + L2);
+    e2 = A.l1 ? fabs(cs - wr) : (cs - wr) * (cs - wr);
+  }
+  A.pot_new[r] = wr > 0.0 ? A.logw2[r] - L2 : -__builtin_inf();
+  A.shift[r] = I;
+  return e2;
+}
+
+// ---------------------------------------------------------------------------
 // MFMA pass.
 struct PassArgs {
   const void* r_pk;
@@ -209,6 +264,8 @@ struct PassArgs {
   int* part_idx;  // max mode: arg max
   int nr_pad, nc_pad;
   const Ctrl* ctrl;
+  OnlineMergeArgs merge;  // LSE mode
+  int* tickets;           // LSE mode: splits done of each block of R points
 };
 
 enum PassMode : int { kModeLse = 0, kModeMax = 1 };
@@ -248,7 +305,7 @@ void online_pass_kernel(PassArgs A) {
   constexpr int es = Op<P>::es;
   constexpr int PARTS = Op<P>::parts;
   constexpr int T = 64 * kWaves;
-  constexpr int SS = Op<P>::stage;
+  constexpr int SS = stage_points(P, D);
   constexpr bool FP8 = P == POTAMD_ONLINE_FP8;
   constexpr int ROWB = D * es + 16;           // LDS bytes per C point (padded)
   constexpr int TILE = SS * ROWB;
@@ -274,9 +331,9 @@ void online_pass_kernel(PassArgs A) {
   const int l32 = lane & 31;
   const int r = blockIdx.x * kRowsPerWG + wave * 32 + l32;
   const int split = blockIdx.y;
-  const int nsteps = (A.nc + SS - 1) / SS;
-  const int step0 = split * A.steps_per_split * (kStep / SS);
-  const int step1 = min(step0 + A.steps_per_split * (kStep / SS), nsteps);
+  const int c_begin = split * A.steps_per_split * kStep;
+  const int c_end = min(A.nc, c_begin + A.steps_per_split * kStep);
+  const int nstages = (c_end - c_begin + SS - 1) / SS;
   const double s2 = MODE == kModeLse ? s2_of(A.cscale, A.reg) : 0.0;
 
   // R operand: half a point per lane, for the whole pass.
@@ -317,20 +374,22 @@ void online_pass_kernel(PassArgs A) {
   float st_sc = 1.f;
   u32x2 st_kp = {0u, 0u};
   auto load = [&](int step) {
-    const int64_t c0 = (int64_t)step * SS;
+    const int64_t c0 = c_begin + (int64_t)step * SS;
 #pragma unroll
     for (int p = 0; p < PARTS; ++p) {
       const char* cp = static_cast<const char*>(A.c_pk) + ((int64_t)p * A.nc_pad + c0) * D * es;
+      // (a stage of 128 may end past the last of a split, which ends at 64s)
+      auto point = [&](int k) { return SS > kStep ? min(k, A.nc_pad - 1 - (int)c0) : k; };
 #pragma unroll
       for (int i = 0; i < NPT; ++i) {
         const int q = tid + T * i;
         if (NCHUNK % T == 0 || q < NCHUNK)
-          st[p][i] = *reinterpret_cast<const u32x4*>(cp + (int64_t)(q / CPR) * D * es + (q % CPR) * 16);
+          st[p][i] = *reinterpret_cast<const u32x4*>(cp + (int64_t)point(q / CPR) * D * es + (q % CPR) * 16);
       }
     }
     if (tid < SS) {
       const int64_t c = c0 + tid;
-      if (c < A.nc) {
+      if (c < c_end) {
         st_v = MODE == kModeLse ? A.c_pot[c] - s2 * A.c_norm[c] : A.c_norm[c];
       } else {
         st_v = -__builtin_inf();
@@ -448,16 +507,16 @@ void online_pass_kernel(PassArgs A) {
     return acc;
   };
 
-  if (step0 < step1) {
-    load(step0);
+  if (nstages > 0) {
+    load(0);
     store(0);
   }
   __syncthreads();
   int buf = 0;
-  for (int step = step0; step < step1; ++step) {
-    const bool more = step + 1 < step1;
+  for (int step = 0; step < nstages; ++step) {
+    const bool more = step + 1 < nstages;
     if (more) load(step + 1);
-#pragma unroll
+#pragma unroll 2
     for (int sb = 0; sb < SS / 32; ++sb) {
       f32x16 t = tile(buf, sb, cl);
       if constexpr (MODE == kModeLse) {
@@ -497,7 +556,7 @@ void online_pass_kernel(PassArgs A) {
         ssum += (double)ts;
       } else {
         const double* vrow = &sm_v[buf][sb * 32 + 4 * h];
-        const int cb = step * SS + sb * 32 + 4 * h;
+        const int cb = c_begin + step * SS + sb * 32 + 4 * h;
 #pragma unroll
         for (int q = 0; q < 4; ++q)
 #pragma unroll
@@ -530,7 +589,36 @@ void online_pass_kernel(PassArgs A) {
     } else {
       I = -__builtin_inf();
     }
-    if (h == 0) A.part[(int64_t)split * A.nr_pad + r] = I;
+    // The last split of these R points to finish merges them all: partials
+    // are written and read past the caches that are not coherent, so no fence
+    // is needed (a launch for the merge took 5 us and the gap before it).
+    const int S = gridDim.y;
+    double* part = A.part + r;
+    if (h == 0)
+      __hip_atomic_store(part + (int64_t)split * A.nr_pad, I, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    __shared__ int last;
+    __builtin_amdgcn_s_waitcnt(0);  // this thread's partial is written
+    __syncthreads();
+    if (tid == 0)
+      last = __hip_atomic_fetch_add(A.tickets + blockIdx.x, 1, __ATOMIC_RELAXED,
+                                    __HIP_MEMORY_SCOPE_AGENT) == S - 1;
+    __syncthreads();
+    if (!last) return;
+    double e2 = 0.0;
+    const int row = blockIdx.x * kRowsPerWG + tid;
+    if (tid < kRowsPerWG && row < A.nr) {
+      const double* pr = A.part + row;
+      e2 = merge_row(A.merge, row, S, [&](int s) {
+        return __hip_atomic_load(pr + (int64_t)s * A.nr_pad, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
+      });
+    }
+    if (tid == 0) A.tickets[blockIdx.x] = 0;  // for the next pass
+    if (A.merge.check && tid < kRowsPerWG) {
+      e2 = wave_sum(e2);
+      if (lane == 0) A.merge.errpart[blockIdx.x * (kRowsPerWG / 64) + wave] = e2;
+    }
   } else {
     const float b_o = __shfl_xor(best, 32, 64);
     const int c_o = __shfl_xor(best_c, 32, 64);
@@ -723,28 +811,7 @@ __global__ __launch_bounds__(256) void online_max_reduce_kernel(MaxReduceArgs A)
 }
 
 // ---------------------------------------------------------------------------
-// Merge of the split partials into the new potential of the R side.
-struct OnlineMergeArgs {
-  const double* part;
-  int S, nr, nr_pad;
-  const double* w;       // weights of the R side
-  const double* logw2;   // log2 of the weights
-  const double* norm;    // |r|^2
-  const double* pot_cur; // current potential of the R side (error only)
-  double* pot_new;
-  double* shift;
-  const double* cscale;
-  double reg;
-  int check, decide, iter, max_iter;
-  int l1;         // error: 1 = sum |marginal - w| (empirical_sinkhorn), 0 = 2-norm
-  int inclusive;  // stop: 1 = err <= stop_thr (empirical_sinkhorn), 0 = err < stop_thr
-  double stop_thr;
-  double* err_hist;
-  int err_cap;
-  double* errpart;
-  Ctrl* ctrl;
-};
-
+// Merge of the fp64 pass's split partials (the MFMA passes merge their own).
 // One wave per workgroup (the R side has 16384 points at the headline size:
 // 256 workgroups fill the chip), the split partials read 8 at a time so their
 // loads overlap.  The stop decision is online_decide_kernel's, launched after
@@ -759,25 +826,7 @@ __global__ __launch_bounds__(kMergeRows) void online_merge_kernel(OnlineMergeArg
   double e2 = 0.0;
   if (r < A.nr) {
     const double* pr = A.part + r;
-    double mx = -__builtin_inf();
-#pragma unroll 8
-    for (int s = 0; s < A.S; ++s) mx = fmax(mx, pr[(int64_t)s * A.nr_pad]);
-    double I = -__builtin_inf();
-    if (mx > -__builtin_inf()) {
-      double acc = 0.0;
-#pragma unroll 8
-      for (int s = 0; s < A.S; ++s) acc += exp2(pr[(int64_t)s * A.nr_pad] - mx);
-      I = mx + log2(acc);
-    }
-    const double s2 = s2_of(A.cscale, A.reg);
-    const double L2 = I - s2 * A.norm[r];
-    const double wr = A.w[r];
-    if (A.check) {
-      const double cs = exp2(A.pot_cur[r] + L2);
-      e2 = A.l1 ? fabs(cs - wr) : (cs - wr) * (cs - wr);
-    }
-    A.pot_new[r] = wr > 0.0 ? A.logw2[r] - L2 : -__builtin_inf();
-    A.shift[r] = I;
+    e2 = merge_row(A, r, A.S, [&](int s) { return pr[(int64_t)s * A.nr_pad]; });
   }
   if (!A.check) return;
   e2 = wave_sum(e2);
@@ -825,8 +874,11 @@ __global__ __launch_bounds__(256) void online_decide_kernel(OnlineMergeArgs A, i
 
 // ---------------------------------------------------------------------------
 // Plan, cost and marginals in fp64: M_rc from the fp32 points in fp64,
-// P_rc = exp(-M_rc / reg + u_r + v_c).  One workgroup per 64 rows sweeps all
-// columns; column sums are fp64 atomics, row sums and cost are per block.
+// P_rc = exp(-M_rc / reg + u_r + v_c).  A workgroup takes 64 rows and one split
+// of the columns; column sums are fp64 atomics, row sums and cost are per
+// block.  Bound by the fp64 exponential: one workgroup over all columns left
+// 5000 rows on 79 of 256 CUs, and 32 coordinates were multiplied whatever d is
+// (5000 x 4000 in 3-D: 503 us, now 85).
 struct OnlinePlanArgs {
   const void* X;
   int64_t ldx;
@@ -842,9 +894,10 @@ struct OnlinePlanArgs {
   const double* yn;
   double* P;         // optional n x ldp
   int64_t ldp;
-  double* rowsum;    // [n]
+  double* rowpart;   // [splits][n]
   double* colsum;    // [m], zeroed
-  double* costpart;  // [blocks]
+  double* costpart;  // [splits][blocks]
+  int tiles_per_split;
 };
 
 __global__ __launch_bounds__(256) void online_plan_kernel(OnlinePlanArgs A) {
@@ -864,7 +917,20 @@ __global__ __launch_bounds__(256) void online_plan_kernel(OnlinePlanArgs A) {
     ur[i] = r < A.n ? A.u[r] : -__builtin_inf();
     xr[i] = r < A.n ? A.xn[r] : 0.0;
   }
-  for (int c0 = 0; c0 < A.m; c0 += 64) {
+  auto load = [&](double (*S)[33], const void* pts, int64_t ld, int p0, int count, int k0) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int e = tid + 256 * q;
+      const int row = e >> 5, k = k0 + (e & 31);
+      S[row][e & 31] =
+          (p0 + row < count && k < A.d) ? coord(pts, (int64_t)(p0 + row) * ld + k, A.x64) : 0.0;
+    }
+  };
+  const bool once = A.d <= 32;  // the rows' coordinates stay in LDS
+  if (once) load(Rs, A.X, A.ldx, r0, A.n, 0);
+  const int c_begin = blockIdx.y * A.tiles_per_split * 64;
+  const int c_end = min(A.m, c_begin + A.tiles_per_split * 64);
+  for (int c0 = c_begin; c0 < c_end; c0 += 64) {
     double acc[4][4];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -872,17 +938,12 @@ __global__ __launch_bounds__(256) void online_plan_kernel(OnlinePlanArgs A) {
       for (int j = 0; j < 4; ++j) acc[i][j] = 0.0;
     for (int k0 = 0; k0 < A.d; k0 += 32) {
       __syncthreads();
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const int e = tid + 256 * q;
-        const int row = e >> 5, col = e & 31;
-        const int k = k0 + col;
-        Rs[row][col] = (r0 + row < A.n && k < A.d) ? coord(A.X, (int64_t)(r0 + row) * A.ldx + k, A.x64) : 0.0;
-        Cs[row][col] = (c0 + row < A.m && k < A.d) ? coord(A.Y, (int64_t)(c0 + row) * A.ldy + k, A.x64) : 0.0;
-      }
+      if (!once) load(Rs, A.X, A.ldx, r0, A.n, k0);
+      load(Cs, A.Y, A.ldy, c0, A.m, k0);
       __syncthreads();
-#pragma unroll 8
-      for (int kk = 0; kk < 32; ++kk) {
+      const int kn = min(32, (A.d - k0 + 3) & ~3);  // (zeros up to there)
+#pragma unroll 4
+      for (int kk = 0; kk < kn; ++kk) {
         double a[4], b[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) a[i] = Rs[ty * 4 + i][kk];
@@ -930,13 +991,24 @@ __global__ __launch_bounds__(256) void online_plan_kernel(OnlinePlanArgs A) {
 #pragma unroll
     for (int o = 1; o < 16; o <<= 1) rs[i] += __shfl_xor(rs[i], o, 64);
     const int r = r0 + ty * 4 + i;
-    if (tx == 0 && r < A.n) A.rowsum[r] = rs[i];
+    if (tx == 0 && r < A.n) A.rowpart[(int64_t)blockIdx.y * A.n + r] = rs[i];
   }
   __shared__ double red[4];
   cost = wave_sum(cost);
   if ((tid & 63) == 0) red[tid >> 6] = cost;
   __syncthreads();
-  if (tid == 0) A.costpart[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
+  if (tid == 0) A.costpart[blockIdx.y * gridDim.x + blockIdx.x] = red[0] + red[1] + red[2] + red[3];
+}
+
+// Row sums from the splits', in a fixed order.
+__global__ __launch_bounds__(256) void online_plan_rows_kernel(int n, int S, const double* rowpart,
+                                                               double* rowsum) {
+  const int r = blockIdx.x * 256 + threadIdx.x;
+  if (r >= n) return;
+  double t = 0.0;
+#pragma unroll 4
+  for (int s = 0; s < S; ++s) t += rowpart[(int64_t)s * n + r];
+  rowsum[r] = t;
 }
 
 // sums = [cost, total mass, ||rowsum - a||_2, ||colsum - b||_2]
@@ -1020,6 +1092,7 @@ struct OnlineLayout {
   double* errpart;
   double* blockmax;
   double* cscale;
+  int* tickets;
   Ctrl* ctrl;
   size_t bytes;
 };
@@ -1060,7 +1133,8 @@ OnlineLayout carve_online(void* ws, int prec, int n, int m, int d) {
   const size_t parts = (size_t)64 * std::max(np, mp);
   L.part = c.take<double>(parts);
   L.pidx = c.take<int>(parts);
-  L.errpart = c.take<double>((std::max(n, m) + kMergeRows - 1) / kMergeRows);
+  L.errpart = c.take<double>(std::max(np, mp) / kMergeRows);
+  L.tickets = c.take<int>(std::max(np, mp) / kRowsPerWG);
   L.blockmax = c.take<double>((std::max(n, m) + 255) / 256);
   L.cscale = c.take<double>(1);
   L.ctrl = c.take<Ctrl>(1);
@@ -1130,6 +1204,19 @@ hipError_t half_step(int prec, int D, int d, const Side& R, const Side& C, const
   const int nsteps = (C.count + kStep - 1) / kStep;
   const int sps = (nsteps + S - 1) / S;
   const int Seff = (nsteps + sps - 1) / sps;
+  ma.part = L.part;
+  ma.S = Seff;
+  ma.nr = R.count;
+  ma.nr_pad = R.pad;
+  ma.w = R.w;
+  ma.logw2 = R.logw2;
+  ma.norm = R.norm;
+  ma.shift = R.shift;
+  ma.cscale = L.cscale;
+  ma.reg = reg;
+  ma.errpart = L.errpart;
+  ma.ctrl = L.ctrl;
+  const int nblk = (R.count + kMergeRows - 1) / kMergeRows;
   if (prec == POTAMD_ONLINE_F64) {
     F64PassArgs fa;
     fa.x64 = R.x64;
@@ -1149,6 +1236,7 @@ hipError_t half_step(int prec, int D, int d, const Side& R, const Side& C, const
     fa.nr_pad = R.pad;
     fa.ctrl = L.ctrl;
     hipLaunchKernelGGL(online_f64_pass_kernel, dim3(R.pad / 64, Seff), dim3(256), 0, s, fa);
+    hipLaunchKernelGGL(online_merge_kernel, dim3(nblk), dim3(kMergeRows), 0, s, ma);
   } else {
     PassArgs pa;
     pa.r_pk = R.pk;
@@ -1168,25 +1256,11 @@ hipError_t half_step(int prec, int D, int d, const Side& R, const Side& C, const
     pa.nr_pad = R.pad;
     pa.nc_pad = C.pad;
     pa.ctrl = L.ctrl;
+    pa.merge = ma;
+    pa.tickets = L.tickets;
     hipError_t e = launch_pass(prec, D, pa, Seff, s);
     if (e != hipSuccess) return e;
   }
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  ma.part = L.part;
-  ma.S = Seff;
-  ma.nr = R.count;
-  ma.nr_pad = R.pad;
-  ma.w = R.w;
-  ma.logw2 = R.logw2;
-  ma.norm = R.norm;
-  ma.shift = R.shift;
-  ma.cscale = L.cscale;
-  ma.reg = reg;
-  ma.errpart = L.errpart;
-  ma.ctrl = L.ctrl;
-  const int nblk = (R.count + kMergeRows - 1) / kMergeRows;
-  hipLaunchKernelGGL(online_merge_kernel, dim3(nblk), dim3(kMergeRows), 0, s, ma);
   if (ma.decide) hipLaunchKernelGGL(online_decide_kernel, dim3(1), dim3(256), 0, s, ma, nblk);
   return hipGetLastError();
 }
@@ -1237,6 +1311,8 @@ extern "C" int potamd_sinkhorn_online(int precision, int dtype, const void* X, i
   HIP_TRY(launch_log2(n, a, L.loga2, s));
   HIP_TRY(launch_log2(m, b, L.logb2, s));
   HIP_TRY(launch_scale_copy(n, u, kLog2e, L.U[0], s));
+  // Tickets start at zero (pairs of them as doubles; there is an even count's room).
+  HIP_TRY(fill((std::max(np, mp) / kRowsPerWG + 1) / 2, 0.0, reinterpret_cast<double*>(L.tickets), s));
   HIP_TRY(fill(np, nan, L.shX, s));
   HIP_TRY(fill(mp, nan, L.shY, s));
 
@@ -1438,16 +1514,39 @@ extern "C" int potamd_sinkhorn_online(int precision, int dtype, const void* X, i
   return status;
 }
 
+namespace {
+// Column splits of the plan kernel: about 2048 workgroups, at most 64.
+int plan_splits(int n, int m, int* tiles_per_split) {
+  const int nblk = (n + 63) / 64, tiles = (m + 63) / 64;
+  int s = std::min(64, std::max(1, std::min(tiles, (2048 + nblk - 1) / nblk)));
+  const int per = (tiles + s - 1) / s;
+  if (tiles_per_split) *tiles_per_split = per;
+  return (tiles + per - 1) / per;
+}
+
+struct OnlinePlanLayout {
+  double *xn, *yn, *rowsum, *colsum, *rowpart, *costpart, *cscale;
+  size_t bytes;
+};
+OnlinePlanLayout carve_online_plan(void* ws, int n, int m) {
+  Carver c(ws);
+  OnlinePlanLayout L;
+  const int S = plan_splits(n, m, nullptr);
+  L.xn = c.take<double>(n);
+  L.yn = c.take<double>(m);
+  L.rowsum = c.take<double>(n);
+  L.colsum = c.take<double>(m);
+  L.rowpart = c.take<double>((size_t)S * n);
+  L.costpart = c.take<double>((size_t)S * ((n + 63) / 64));
+  L.cscale = c.take<double>(1);
+  L.bytes = c.off;
+  return L;
+}
+}  // namespace
+
 extern "C" size_t potamd_online_plan_workspace_size(int n, int m) {
   if (n < 1 || m < 1) return 0;
-  Carver c(nullptr);
-  c.take<double>(n);                 // xn
-  c.take<double>(m);                 // yn
-  c.take<double>(n);                 // rowsum
-  c.take<double>(m);                 // colsum
-  c.take<double>((n + 63) / 64);     // costpart
-  c.take<double>(1);                 // cscale
-  return c.off;
+  return carve_online_plan(nullptr, n, m).bytes;
 }
 
 extern "C" int potamd_online_plan(int dtype, const void* X, int64_t ldx, const void* Y, int64_t ldy, int n,
@@ -1460,17 +1559,11 @@ extern "C" int potamd_online_plan(int dtype, const void* X, int64_t ldx, const v
       (dtype != POTAMD_F32 && dtype != POTAMD_F64))
     return POTAMD_EINVAL;
   const int x64 = dtype == POTAMD_F64;
-  Carver c(workspace);
-  double* xn = c.take<double>(n);
-  double* yn = c.take<double>(m);
-  double* rowsum = c.take<double>(n);
-  double* colsum = c.take<double>(m);
-  double* costpart = c.take<double>((n + 63) / 64);
-  double* cscale = c.take<double>(1);
-  if (!workspace || ws_bytes < c.off) return POTAMD_EWORKSPACE;
+  const OnlinePlanLayout L = carve_online_plan(workspace, n, m);
+  if (!workspace || ws_bytes < L.bytes) return POTAMD_EWORKSPACE;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  HIP_TRY(fill(1, cost_scale, cscale, s));
-  HIP_TRY(fill(m, 0.0, colsum, s));
+  HIP_TRY(fill(1, cost_scale, L.cscale, s));
+  HIP_TRY(fill(m, 0.0, L.colsum, s));
   PackArgs pk;
   memset(&pk, 0, sizeof(pk));
   pk.d = d;
@@ -1480,13 +1573,13 @@ extern "C" int potamd_online_plan(int dtype, const void* X, int64_t ldx, const v
   pk.ldx = ldx;
   pk.rows = n;
   pk.rows_pad = n;
-  pk.norms = xn;
+  pk.norms = L.xn;
   HIP_TRY(launch_pack(POTAMD_ONLINE_F64, pk, s));
   pk.X = Y;
   pk.ldx = ldy;
   pk.rows = m;
   pk.rows_pad = m;
-  pk.norms = yn;
+  pk.norms = L.yn;
   HIP_TRY(launch_pack(POTAMD_ONLINE_F64, pk, s));
   OnlinePlanArgs pa;
   pa.x64 = x64;
@@ -1498,21 +1591,24 @@ extern "C" int potamd_online_plan(int dtype, const void* X, int64_t ldx, const v
   pa.m = m;
   pa.d = d;
   pa.reg = reg;
-  pa.cscale = cscale;
+  pa.cscale = L.cscale;
   pa.u = u;
   pa.v = v;
-  pa.xn = xn;
-  pa.yn = yn;
+  pa.xn = L.xn;
+  pa.yn = L.yn;
   pa.P = P;
   pa.ldp = ldp;
-  pa.rowsum = rowsum;
-  pa.colsum = colsum;
-  pa.costpart = costpart;
+  pa.rowpart = L.rowpart;
+  pa.colsum = L.colsum;
+  pa.costpart = L.costpart;
   const int nblk = (n + 63) / 64;
-  hipLaunchKernelGGL(online_plan_kernel, dim3(nblk), dim3(256), 0, s, pa);
+  const int S = plan_splits(n, m, &pa.tiles_per_split);
+  hipLaunchKernelGGL(online_plan_kernel, dim3(nblk, S), dim3(256), 0, s, pa);
+  hipLaunchKernelGGL(online_plan_rows_kernel, dim3((n + 255) / 256), dim3(256), 0, s, n, S,
+                     L.rowpart, L.rowsum);
   HIP_TRY(hipGetLastError());
-  hipLaunchKernelGGL(online_plan_final_kernel, dim3(1), dim3(256), 0, s, n, m, nblk, rowsum,
-                     colsum, costpart, a, b, sums);
+  hipLaunchKernelGGL(online_plan_final_kernel, dim3(1), dim3(256), 0, s, n, m, nblk * S,
+                     L.rowsum, L.colsum, L.costpart, a, b, sums);
   HIP_TRY(hipGetLastError());
   return POTAMD_CONVERGED;
 }
