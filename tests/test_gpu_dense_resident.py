@@ -129,6 +129,30 @@ def test_references_and_exact_rows(n, m, reg, zeros, dtype):
             assert (x[fin] - y[fin]).abs().max().item() < max(tol, 2e-5 if dtype == F32 else 0.0)
 
 
+@pytest.mark.parametrize("n,m,dtype", [(4801, 4500, F32), (5120, 5119, F32), (2816, 2900, F64)])
+def test_largest_blocks(n, m, dtype):
+    """Every CU holds a block; against the row sweep."""
+    g = torch.Generator(device="cuda").manual_seed(n)
+    M = torch.rand((1, n, m), generator=g, device="cuda", dtype=dtype)
+    a = torch.rand((1, n), generator=g, device="cuda", dtype=torch.float64) + 0.2
+    b = torch.rand((1, m), generator=g, device="cuda", dtype=torch.float64) + 0.2
+    a, b = a / a.sum(), b / b.sum()
+    assert _lib.load().potamd_dense_resident(_lib.F32 if dtype == F32 else _lib.F64, 1, n, m)
+    tile = (1024, 8, 0, 1) if dtype == F32 else (1024, 4, 0, 1)
+    for domain in (_lib.LOG, _lib.SCALING):
+        u0, v0 = torch.zeros_like(a), torch.zeros_like(b)
+        if domain == _lib.SCALING:
+            u0, v0 = torch.full_like(a, 1.0 / n), torch.full_like(b, 1.0 / m)
+        kw = dict(domain=domain, order=_lib.COL_FIRST, max_iter=12, stop_thr=0.0)
+        want = _solve.dense_solve(M, a, b, u0, v0, 0.05, tile=tile, **kw)
+        got = _solve.dense_solve(M, a, b, u0, v0, 0.05, **kw)
+        for x, y in ((got.u, want.u), (got.v, want.v)):
+            if domain == _lib.SCALING:
+                x, y = torch.log(x), torch.log(y)
+            # 12 iterations of sums of 5000 terms
+            assert (x - y).abs().max().item() < (1e-11 if dtype == F64 else 5e-6)
+
+
 @pytest.mark.parametrize("dtype", [F64, F32])
 @pytest.mark.parametrize("B,n,m", [(2100, 30, 40), (5, 300, 260)])
 def test_each_problem_stops_itself(B, n, m, dtype):
