@@ -73,7 +73,21 @@ def _load():
 def lookup(dtype, n, m):
     """Cached (threads, cols_per_thread, rows_per_block, prefetch) or None."""
     ent = _load().get(_key(dtype, n, m))
-    return tuple(ent["tile"]) if ent else None
+    if not ent:
+        return None
+    tile = tuple(ent["tile"])
+    n0, m0 = ent.get("n"), ent.get("m")
+    if not n0 or not m0 or not tile[2]:
+        return tile
+    # A row well short of the timed one leaves much of the tile empty, and another
+    # may be faster: 14000^2 float32 153 us an iteration with the tile of 16384^2,
+    # 144 with the default; 15000 wide, 177.5 and 176; 16000 wide, 175 and 182.
+    if 8 * int(m) < 7 * m0:
+        return None
+    # The rows a workgroup, scaled from the n that was timed, so that the number
+    # of workgroups is kept: 64 rows at n = 12000 of the 16384 class left 68 of
+    # the 256 CUs idle (12000^2 float32 152 us an iteration, 122 at 47 rows).
+    return tile[:2] + (min(256, max(4, -(-tile[2] * int(n) // n0))),) + tile[3:]
 
 
 def candidates(dtype, m):
@@ -118,7 +132,8 @@ def tune(n, m, dtype="f32", iters=20, reps=2, save=True, log=None):
     if save:
         with _lock:
             mem = _load()
-            mem[_key(dtype, n, m)] = {"tile": list(best_tile), "us_per_iter": best_t * 1e6,
+            mem[_key(dtype, n, m)] = {"tile": list(best_tile), "n": int(n), "m": int(m),
+                                      "us_per_iter": best_t * 1e6,
                                       "measured": [[t * 1e6, list(c)] for t, c in results]}
             with open(CACHE, "w") as fh:
                 json.dump(mem, fh, indent=1, sort_keys=True)

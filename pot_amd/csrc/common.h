@@ -30,7 +30,7 @@ struct Ctrl {
   int bad_iter;    // scaling domain: iteration whose update produced 0/nan/inf
   unsigned counter;  // last-block-done ticket of the merge kernel (self-resetting)
   int n_err;       // number of err values written
-  int need_exact;  // log domain: a column mass fell below the trusted range
+  int need_exact;  // log domain: 1 + the iteration whose column mass fell below the trusted range
   int pad1;
   double err;      // last marginal error
 };

@@ -50,13 +50,17 @@ __device__ __forceinline__ R block_max(R x, R* red, int& parity) {
   return s;
 }
 
-// Vector of VEC elements loaded with one 16-byte (or scalar) access.
+// Vector of VEC elements loaded with one 16-byte (or scalar) access.  Its
+// alignment is the element's: rows of any stride are read 16 bytes at a time
+// (4-byte loads of a 5000 x 4999 float32 cost took 61 us an iteration, 16-byte
+// ones 49).
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef double f64x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef double f64x2u __attribute__((ext_vector_type(2), aligned(8)));
 template <typename TM, int VEC> struct VecT;
-template <> struct VecT<float, 4> { using type = f32x4; };
+template <> struct VecT<float, 4> { using type = f32x4u; };
 template <> struct VecT<float, 1> { using type = float; };
-template <> struct VecT<double, 2> { using type = f64x2; };
+template <> struct VecT<double, 2> { using type = f64x2u; };
 template <> struct VecT<double, 1> { using type = double; };
 
 template <typename TM, int VEC>
@@ -110,12 +114,20 @@ __global__ __launch_bounds__(T) void row_sweep_kernel(RowSweepArgs A) {
   R acc[CPT];
 #pragma unroll
   for (int q = 0; q < CPT; ++q) acc[q] = 0;
+  // Slot j of the block's T * CPT columns is column j, but the vector that
+  // would end past the row is the row's last VEC columns, and its slots before
+  // its own start belong to its neighbour (m >= VEC).
+  auto column = [&](int j0, int c) {  // of slot j0 + c, j0 a vector's start; or -1
+    if (j0 + VEC <= m) return j0 + c;
+    const int col = m - VEC + c;
+    return j0 < m && col >= j0 ? col : -1;
+  };
   for (int j = tid; j < T * CPT; j += T) {
-    const bool ok = j < m;
+    const int col = column(j - j % VEC, j % VEC);
     if (DOMAIN == kLog)
-      vsh[j] = ok ? vp[j] : -__builtin_inf();
+      vsh[j] = col >= 0 ? vp[col] : -__builtin_inf();
     else
-      vsh[j] = ok ? vp[j] : 0.0;
+      vsh[j] = col >= 0 ? vp[col] : 0.0;
   }
   __syncthreads();
   auto vcol = [&](int q) -> double {
@@ -159,7 +171,7 @@ __global__ __launch_bounds__(T) void row_sweep_kernel(RowSweepArgs A) {
     for (int k = 0; k < NCH; ++k) {
       const int j0 = (k * T + tid) * VEC;
       TM tmp[VEC];
-      load_vec<TM, VEC>(row + (j0 < m ? j0 : 0), tmp);
+      load_vec<TM, VEC>(row + (j0 + VEC <= m ? j0 : (j0 < m ? m - VEC : 0)), tmp);
 #pragma unroll
       for (int c = 0; c < VEC; ++c) dst[k * VEC + c] = (R)tmp[c];
     }
@@ -274,8 +286,8 @@ __global__ __launch_bounds__(T) void row_sweep_kernel(RowSweepArgs A) {
   for (int k = 0; k < NCH; ++k) {
 #pragma unroll
     for (int c = 0; c < VEC; ++c) {
-      const int j = (k * T + tid) * VEC + c;
-      if (j < m) cp[j] = acc[k * VEC + c];
+      const int j = column((k * T + tid) * VEC, c);
+      if (j >= 0) cp[j] = acc[k * VEC + c];
     }
   }
   if (MODE == 1) return;
@@ -422,7 +434,7 @@ __global__ __launch_bounds__(256) void col_merge_kernel(MergeArgs A) {
   if (tid == 0) {
     A.errpart[(int64_t)p * gridDim.x + blockIdx.x] = red[0] + red[1] + red[2] + red[3];
     if (any_bad) A.bad[next_slot] = 1;
-    if (any_exact) atomicOr(&ctrl->need_exact, 1);
+    if (any_exact) atomicCAS(&ctrl->need_exact, 0, A.iter + 1);
   }
 }
 
@@ -456,7 +468,7 @@ __global__ __launch_bounds__(256) void col_decide_kernel(MergeArgs A) {
       if (tid == 0) {
         ctrl->done = 1;
         ctrl->status = kNeedExact;
-        ctrl->niter = it;
+        ctrl->niter = need_exact - 1;
       }
       return;
     }
@@ -530,7 +542,7 @@ __global__ __launch_bounds__(256) void col_decide_kernel(MergeArgs A) {
   if (ctrl->need_exact) {
     ctrl->done = 1;
     ctrl->status = kNeedExact;
-    ctrl->niter = it;
+    ctrl->niter = ctrl->need_exact - 1;
     return;
   }
   if (check_col || check_row) {
@@ -560,53 +572,126 @@ __global__ __launch_bounds__(256) void col_decide_kernel(MergeArgs A) {
 }
 
 // Exact column log-sum-exp in base 2 (prologue of the log domain,
-// v1 = log b - LSE_i(Mr + u0), ot/bregman/_sinkhorn.py:881 at ii = 0).
-// One column per thread, rows split over gridDim.y blocks; online
-// (max, sum) in fp64.
+// v1 = log b - LSE_i(Mr + u0), ot/bregman/_sinkhorn.py:881 at ii = 0), in fp64.
+// A thread owns VEC adjacent columns of A.rpb rows and takes eight rows at a
+// time: their loads together, their maximum, one rescaling of the sum, eight
+// exponentials.  (A column and a row at a time, each load waited for and the
+// sum rescaled on every new maximum, took 504 us at 16384^2 float32; 279
+// now, against 170 us to read the cost.)
 
-template <typename TM>
-__global__ __launch_bounds__(256) void col_lse_partial_kernel(ColLseArgs A) {
-  const int p = blockIdx.z, g = blockIdx.y, G = gridDim.y;
-  const int j = blockIdx.x * 256 + threadIdx.x;
-  if (j >= A.m) return;
-  const TM* Mp = static_cast<const TM*>(A.M) + (int64_t)p * A.bstride;
-  const double* u = A.u2 + (int64_t)p * A.n;
-  const int r0 = g * A.rpb, r1 = min(A.n, r0 + A.rpb);
-  double mx = -__builtin_inf(), sm = 0.0;
-  for (int i = r0; i < r1; ++i) {
-    const double x = (double)Mp[(int64_t)i * A.ldm + j] * A.s2 + u[i];
-    if (x == -__builtin_inf()) continue;
-    if (x > mx) {
-      sm = sm * exp2(mx - x) + 1.0;
-      mx = x;
-    } else {
-      sm += exp2(x - mx);
-    }
-  }
-  const int64_t o = ((int64_t)p * G + g) * A.m + j;
-  A.pmax[o] = mx;
-  A.psum[o] = sm;
+// 2^x for x <= 0 to fp64 accuracy: the polynomial interpolates 2^r on
+// [-1/2, 1/2] at 12 Chebyshev nodes (3e-18 off).  -inf gives 0, a NaN stays.
+__device__ __forceinline__ double exp2_neg(double x) {
+  x = x < -1100.0 ? -1100.0 : x;
+  const double k = rint(x), r = x - k;
+  double y = 4.4558179083360645e-10;
+  y = fma(y, r, 7.074194297288521e-09);
+  y = fma(y, r, 1.0178057087733941e-07);
+  y = fma(y, r, 1.3215432535912375e-06);
+  y = fma(y, r, 1.5252733841556773e-05);
+  y = fma(y, r, 0.00015403530463724353);
+  y = fma(y, r, 0.001333355814640647);
+  y = fma(y, r, 0.009618129107587256);
+  y = fma(y, r, 0.055504108664821625);
+  y = fma(y, r, 0.24022650695910158);
+  y = fma(y, r, 0.6931471805599453);
+  y = fma(y, r, 1.0);
+  return ldexp(y, (int)k);
 }
 
+template <typename TM, int VEC>
+__global__ __launch_bounds__(256) void col_lse_partial_kernel(ColLseArgs A) {
+  const int p = blockIdx.z, g = blockIdx.y, G = gridDim.y;
+  const int j0 = (blockIdx.x * 256 + threadIdx.x) * VEC;
+  if (j0 >= A.m) return;
+  const int js = min(j0, A.m - VEC);  // the last vector ends with the row
+  const TM* Mp = static_cast<const TM*>(A.M) + (int64_t)p * A.bstride + js;
+  const double* u = A.u2 + (int64_t)p * A.n;
+  const int r0 = g * A.rpb, r1 = min(A.n, r0 + A.rpb);
+  constexpr int Q = 8;
+  double mx[VEC], sm[VEC];
+#pragma unroll
+  for (int c = 0; c < VEC; ++c) {
+    mx[c] = -__builtin_inf();
+    sm[c] = 0.0;
+  }
+  for (int i = r0; i < r1; i += Q) {
+    TM x[Q][VEC];
+    double ui[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const int r = min(i + q, r1 - 1);
+      load_vec<TM, VEC>(Mp + (int64_t)r * A.ldm, x[q]);
+      ui[q] = i + q < r1 ? u[r] : -__builtin_inf();
+    }
+#pragma unroll
+    for (int c = 0; c < VEC; ++c) {
+      double t[Q], top = mx[c];
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        t[q] = fma((double)x[q][c], A.s2, ui[q]);
+        top = t[q] > top ? t[q] : top;
+      }
+      if (top == -__builtin_inf()) {
+        bool nan = false;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) nan = nan || t[q] != t[q];
+        if (!nan) continue;
+      }
+      sm[c] *= exp2_neg(mx[c] - top);
+      mx[c] = top;
+#pragma unroll
+      for (int q = 0; q < Q; ++q) sm[c] += exp2_neg(t[q] - top);
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < VEC; ++c) {
+    if (js + c < j0) continue;  // the neighbour's
+    const int64_t o = ((int64_t)p * G + g) * A.m + js + c;
+    A.pmax[o] = mx[c];
+    A.psum[o] = sm[c];
+  }
+}
+
+// 64 columns a block, four groups of row blocks each.
 __global__ __launch_bounds__(256) void col_lse_merge_kernel(int m, int G, const double* pmax,
                                                             const double* psum,
                                                             const double* logb2, double* v_out) {
   const int p = blockIdx.y;
-  const int j = blockIdx.x * 256 + threadIdx.x;
-  if (j >= m) return;
-  double mx = -__builtin_inf();
-  for (int g = 0; g < G; ++g) {
-    const double x = pmax[((int64_t)p * G + g) * m + j];
-    mx = x > mx ? x : mx;
-  }
-  double sm = 0.0;
-  if (mx != -__builtin_inf()) {
-    for (int g = 0; g < G; ++g) {
-      const int64_t o = ((int64_t)p * G + g) * m + j;
-      sm += psum[o] * exp2(pmax[o] - mx);
+  const int cl = threadIdx.x & 63, grp = threadIdx.x >> 6;
+  const int j = blockIdx.x * 64 + cl;
+  const int per = (G + 3) / 4, g0 = grp * per, g1 = min(G, g0 + per);
+  double mx = -__builtin_inf(), sm = 0.0;
+  if (j < m) {
+    const double* pm = pmax + (int64_t)p * G * m + j;
+    const double* ps = psum + (int64_t)p * G * m + j;
+#pragma unroll 8
+    for (int g = g0; g < g1; ++g) {
+      const double x = pm[(int64_t)g * m];
+      mx = x > mx ? x : mx;
+    }
+    if (mx != -__builtin_inf()) {
+#pragma unroll 8
+      for (int g = g0; g < g1; ++g) sm += ps[(int64_t)g * m] * exp2(pm[(int64_t)g * m] - mx);
+    } else {
+      for (int g = g0; g < g1; ++g) sm += ps[(int64_t)g * m];  // 0, or a NaN
     }
   }
-  const double lse = mx + log2(sm);
+  __shared__ double smx[4][64], ssm[4][64];
+  smx[grp][cl] = mx;
+  ssm[grp][cl] = sm;
+  __syncthreads();
+  if (grp != 0 || j >= m) return;
+  double top = smx[0][cl];
+#pragma unroll
+  for (int g = 1; g < 4; ++g) top = smx[g][cl] > top ? smx[g][cl] : top;
+  double tot = 0.0;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const double s = ssm[g][cl];
+    tot += top != -__builtin_inf() && s != 0.0 ? s * exp2(smx[g][cl] - top) : s;
+  }
+  const double lse = top + log2(tot);
   v_out[(int64_t)p * m + j] = logb2[(int64_t)p * m + j] - lse;
 }
 
@@ -729,7 +814,7 @@ struct RowCfg {
 // Tile shapes compiled per dtype; the default for m is the first entry that
 // covers it (the autotuner may pick any entry that covers m).
 const RowCfg kRowF32[] = {{64, 4, 1},    {256, 4, 1},   {256, 8, 1},  {512, 8, 1},
-                          {1024, 8, 1},  {1024, 16, 1}, {1024, 8, 2}, {1024, 16, 2},
+                          {1024, 8, 1},  {1024, 16, 2}, {1024, 8, 2}, {1024, 16, 1},
                           {512, 32, 1},  {512, 32, 2}};
 const RowCfg kRowF64[] = {{64, 2, 1},  {256, 2, 1},  {256, 4, 1},
                           {512, 4, 1}, {1024, 4, 1}, {1024, 8, 1}};
@@ -776,20 +861,34 @@ hipError_t launch_col_merge(int dtype, const MergeArgs& a, int B, hipStream_t s)
     hipLaunchKernelGGL(col_merge_kernel<float>, grid, dim3(256), 0, s, a);
   else
     hipLaunchKernelGGL(col_merge_kernel<double>, grid, dim3(256), 0, s, a);
-  if (!a.prologue) hipLaunchKernelGGL(col_decide_kernel, dim3(1), dim3(256), 0, s, a);
+  // The log domain decides only where it checks and at the end (a column mass
+  // off the range is kept with its iteration); the scaling domain's guard
+  // looks at every iteration.  5 us and the gap before it, of 188 us at 16384^2.
+  const int it = a.iter;
+  const bool check = a.order == kColFirst ? it % 10 == 0 : it >= 1 && (it - 1) % 10 == 0;
+  if (!a.prologue && (a.domain == kScaling || check || it >= a.max_iter - 1))
+    hipLaunchKernelGGL(col_decide_kernel, dim3(1), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
 hipError_t launch_col_lse(int dtype, const ColLseArgs& a, int G, int B, const double* logb2,
                           double* v_out, hipStream_t s) {
-  dim3 grid((a.m + 255) / 256, G, B);
-  if (dtype == 0)
-    hipLaunchKernelGGL(col_lse_partial_kernel<float>, grid, dim3(256), 0, s, a);
-  else
-    hipLaunchKernelGGL(col_lse_partial_kernel<double>, grid, dim3(256), 0, s, a);
+  const int vec = dtype == 0 ? (a.m >= 4 ? 4 : 1) : (a.m >= 2 ? 2 : 1);
+  dim3 grid((a.m + 256 * vec - 1) / (256 * vec), G, B);
+  if (dtype == 0) {
+    if (vec == 4)
+      hipLaunchKernelGGL((col_lse_partial_kernel<float, 4>), grid, dim3(256), 0, s, a);
+    else
+      hipLaunchKernelGGL((col_lse_partial_kernel<float, 1>), grid, dim3(256), 0, s, a);
+  } else {
+    if (vec == 2)
+      hipLaunchKernelGGL((col_lse_partial_kernel<double, 2>), grid, dim3(256), 0, s, a);
+    else
+      hipLaunchKernelGGL((col_lse_partial_kernel<double, 1>), grid, dim3(256), 0, s, a);
+  }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(col_lse_merge_kernel, dim3((a.m + 255) / 256, B), dim3(256), 0, s, a.m, G,
+  hipLaunchKernelGGL(col_lse_merge_kernel, dim3((a.m + 63) / 64, B), dim3(256), 0, s, a.m, G,
                      a.pmax, a.psum, logb2, v_out);
   return hipGetLastError();
 }
