@@ -12,8 +12,10 @@
 //   the squared Euclidean cost.
 //
 // Both are small next to the Sinkhorn sweeps (they run once per solve or
-// once per outer Gromov step); they are written for correctness and full
-// occupancy rather than MFMA peak: 256 threads, 4 x 4 outputs per thread.
+// once per outer Gromov step): pairwise_kernel has 256 threads with 4 x 4
+// outputs each, gemm_batched_kernel a short chain on the matrix cores.
+#include <algorithm>
+
 #include "../../include/pot_amd.h"
 #include "host.h"
 #include "internal.h"
@@ -117,12 +119,41 @@ struct GemmBatchArgs {
   double alpha, beta;
 };
 
-template <typename T>
+// One 16 x 16 x 4 step of the matrix core: a = A[lane % 16][lane / 16],
+// b = B[lane / 16][lane % 16]; value i of c is column lane % 16 and row
+// out_row(i) of the product.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+template <typename T> struct Mma;
+template <> struct Mma<float> {
+  using Acc = f32x4;
+  static __device__ __forceinline__ f32x4 step(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int out_row(int lane, int i) { return 4 * (lane / 16) + i; }
+};
+template <> struct Mma<double> {
+  using Acc = f64x4;
+  static __device__ __forceinline__ f64x4 step(double a, double b, f64x4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int out_row(int lane, int i) { return lane / 16 + 4 * i; }
+};
+
+// A workgroup of four waves forms a TS x TS tile of C_b, KC of K at a time
+// through LDS, the next chunk's loads issued before the products of this one.
+// These products are small (K of 40 to a few hundred), so the time is their
+// chain: launch, loads, products, store.  One chunk covers K <= 64 with the
+// tile of 32, which also gives four times the workgroups of the tile of 64.
+template <typename T, int TS, int KC>
 __global__ __launch_bounds__(256) void gemm_batched_kernel(GemmBatchArgs g) {
-  __shared__ T as[kChunk][kTile + 1];
-  __shared__ T bs[kChunk][kTile + 1];
-  const int i0 = blockIdx.y * kTile, j0 = blockIdx.x * kTile;
-  const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
+  __shared__ T as[KC][TS + 1];
+  __shared__ T bs[KC][TS + 1];
+  constexpr int L = TS * KC / 256;  // elements a thread loads of each operand
+  constexpr int SUB = TS / 32;      // 16 x 16 products a side of a wave's quarter
+  const int i0 = blockIdx.y * TS, j0 = blockIdx.x * TS;
+  const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+  const int wi = wave / 2 * (TS / 2), wj = wave % 2 * (TS / 2);
   const T* A = static_cast<const T*>(g.A);
   const T* Bm = static_cast<const T*>(g.Bm);
   T* C = static_cast<T*>(g.C);
@@ -133,66 +164,88 @@ __global__ __launch_bounds__(256) void gemm_batched_kernel(GemmBatchArgs g) {
   for (int b = blockIdx.z; b < g.B; b += gridDim.z) {
     const T* Ab = A + (int64_t)b * g.sA;
     const T* Bb = Bm + (int64_t)b * g.sB;
-    T acc[4][4] = {};
-    for (int k0 = 0; k0 < g.K; k0 += kChunk) {
-      for (int e = threadIdx.x; e < kChunk * kTile; e += 256) {
-        int r, k;
-        if (a_k_fast) {
-          r = e / kChunk;
-          k = e % kChunk;
-        } else {
-          r = e % kTile;
-          k = e / kTile;
-        }
-        const int i = i0 + r, kk = k0 + k;
-        as[k][r] = (i < g.M && kk < g.K) ? Ab[(int64_t)i * g.rsA + (int64_t)kk * g.csA] : (T)0;
-        int c, kb;
-        if (b_j_fast) {
-          c = e % kTile;
-          kb = e / kTile;
-        } else {
-          c = e / kChunk;
-          kb = e % kChunk;
-        }
-        const int j = j0 + c, kk2 = k0 + kb;
-        bs[kb][c] = (j < g.N && kk2 < g.K) ? Bb[(int64_t)kk2 * g.rsB + (int64_t)j * g.csB] : (T)0;
+    T ra[L], rb[L];
+    auto load = [&](int k0) {
+#pragma unroll
+      for (int e = 0; e < L; ++e) {
+        const int q = tid + 256 * e;
+        const int r = a_k_fast ? q / KC : q % TS, k = k0 + (a_k_fast ? q % KC : q / TS);
+        const int i = i0 + r;
+        ra[e] = (i < g.M && k < g.K) ? Ab[(int64_t)i * g.rsA + (int64_t)k * g.csA] : (T)0;
+      }
+#pragma unroll
+      for (int e = 0; e < L; ++e) {
+        const int q = tid + 256 * e;
+        const int c = b_j_fast ? q % TS : q / KC, k = k0 + (b_j_fast ? q / TS : q % KC);
+        const int j = j0 + c;
+        rb[e] = (j < g.N && k < g.K) ? Bb[(int64_t)k * g.rsB + (int64_t)j * g.csB] : (T)0;
+      }
+    };
+    typename Mma<T>::Acc acc[SUB][SUB] = {};
+    load(0);
+    for (int k0 = 0; k0 < g.K; k0 += KC) {
+#pragma unroll
+      for (int e = 0; e < L; ++e) {
+        const int q = tid + 256 * e;
+        as[a_k_fast ? q % KC : q / TS][a_k_fast ? q / KC : q % TS] = ra[e];
+        bs[b_j_fast ? q / TS : q % KC][b_j_fast ? q % TS : q / KC] = rb[e];
       }
       __syncthreads();
+      if (k0 + KC < g.K) load(k0 + KC);
+      const int kn = min(KC, g.K - k0);
+      for (int k = 0; k < kn; k += 4) {  // (rows past K are zero)
+        T av[SUB], bv[SUB];
 #pragma unroll
-      for (int k = 0; k < kChunk; ++k) {
-        T av[4], bv[4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          av[t] = as[k][ty + 16 * t];
-          bv[t] = bs[k][tx + 16 * t];
+        for (int t = 0; t < SUB; ++t) {
+          av[t] = as[k + lane / 16][wi + 16 * t + lane % 16];
+          bv[t] = bs[k + lane / 16][wj + 16 * t + lane % 16];
         }
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
+        for (int r = 0; r < SUB; ++r)
 #pragma unroll
-          for (int c = 0; c < 4; ++c) acc[r][c] = fma(av[r], bv[c], acc[r][c]);
+          for (int c = 0; c < SUB; ++c) acc[r][c] = Mma<T>::step(av[r], bv[c], acc[r][c]);
       }
       __syncthreads();
     }
     T* Cb = C + (int64_t)b * g.sC;
     const T alpha = (T)g.alpha, beta = (T)g.beta;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int i = i0 + ty + 16 * r;
-      if (i >= g.M) continue;
+    for (int r = 0; r < SUB; ++r)
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const int j = j0 + tx + 16 * c;
+      for (int c = 0; c < SUB; ++c) {
+        const int j = j0 + wj + 16 * c + lane % 16;
         if (j >= g.N) continue;
-        T* dst = Cb + (int64_t)i * g.ldc + j;
-        // beta == 0 never reads C, so an uninitialised C stays harmless
-        *dst = beta == (T)0 ? alpha * acc[r][c] : fma(alpha, acc[r][c], beta * *dst);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int i = i0 + wi + 16 * r + Mma<T>::out_row(lane, q);
+          if (i >= g.M) continue;
+          T* dst = Cb + (int64_t)i * g.ldc + j;
+          // beta == 0 never reads C, so an uninitialised C stays harmless
+          *dst = beta == (T)0 ? alpha * acc[r][c][q] : fma(alpha, acc[r][c][q], beta * *dst);
+        }
       }
-    }
   }
 }
 
-dim3 tile_grid(int rows, int cols, int B) {
-  return dim3((cols + kTile - 1) / kTile, (rows + kTile - 1) / kTile, B < 65535 ? B : 65535);
+dim3 tile_grid(int rows, int cols, int B, int tile = kTile) {
+  return dim3((cols + tile - 1) / tile, (rows + tile - 1) / tile, B < 65535 ? B : 65535);
+}
+
+// The tile of 64 (half the loads an output) where its workgroups fill the chip,
+// unless the whole product fits the tile of 32.  us with 64 / 32: 256 float64
+// products of 64^3 8.3 / 11.7 (16 before, with vector instructions), 64 float32
+// of 180 x 8 x 200 (192 tiles of 64) 12.7 / 9.6 (33), 8 float64 of 200^3 (128)
+// 17 / 12 (41), 16 float64 of 48 x 40 x 48 6.4 / 3.7 (10), 4000 float32 of 20^3
+// 28 / 19 (21).
+template <typename T>
+void launch_gemm(const GemmBatchArgs& g, hipStream_t s) {
+  const int64_t wide = (int64_t)((g.M + 63) / 64) * ((g.N + 63) / 64) * g.B;
+  if (wide >= 256 && std::max(g.M, g.N) > 32)
+    hipLaunchKernelGGL((gemm_batched_kernel<T, 64, 32>), tile_grid(g.M, g.N, g.B, 64), dim3(256), 0,
+                       s, g);
+  else
+    hipLaunchKernelGGL((gemm_batched_kernel<T, 32, 64>), tile_grid(g.M, g.N, g.B, 32), dim3(256), 0,
+                       s, g);
 }
 
 }  // namespace
@@ -238,11 +291,10 @@ extern "C" int potamd_gemm_batched(int dtype, int batch, int M, int N, int K, do
     return POTAMD_EINVAL;
   GemmBatchArgs g{batch, M, N, K, A, sA, rsA, csA, B, sB, rsB, csB, C, sC, ldc, alpha, beta};
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const dim3 grid = tile_grid(M, N, batch);
   if (dtype == POTAMD_F32)
-    hipLaunchKernelGGL(gemm_batched_kernel<float>, grid, dim3(256), 0, s, g);
+    launch_gemm<float>(g, s);
   else
-    hipLaunchKernelGGL(gemm_batched_kernel<double>, grid, dim3(256), 0, s, g);
+    launch_gemm<double>(g, s);
   HIP_TRY(hipGetLastError());
   return 0;
 }
