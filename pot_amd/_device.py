@@ -28,16 +28,34 @@ def require_gpu():
 
 
 def stream_ptr(device):
-    return torch.cuda.current_stream(device).cuda_stream
+    """Handle of the current stream (as an integer: building the Stream object
+    took 5 us a call, more than most of the launches it was for)."""
+    idx = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if idx is None else idx)
+
+
+_CTRL_BYTES = 1024
+_HOST_ERRS = 8192
 
 
 def host_ctrl():
-    """Per-thread pinned host buffer used by the solver's stop polling."""
+    """Per-thread pinned host buffer: the solver's stop polling, then room for
+    the errors of one solve."""
     buf = getattr(_tls, "ctrl", None)
     if buf is None:
-        buf = torch.zeros(1024, dtype=torch.uint8, pin_memory=True)
+        buf = torch.zeros(_CTRL_BYTES + 8 * _HOST_ERRS, dtype=torch.uint8, pin_memory=True)
         _tls.ctrl = buf
     return buf
+
+
+def err_buffer(cap, device):
+    """Room for ``cap`` error values of one solve.  The kernels write them into
+    this thread's pinned memory, which a solve that waits for its result reads
+    without a copy (clearing and copying a device buffer took 25 us a solve);
+    a longer history has a buffer on the device."""
+    if cap > _HOST_ERRS:
+        return torch.zeros(cap, dtype=torch.float64, device=device)
+    return host_ctrl()[_CTRL_BYTES:_CTRL_BYTES + 8 * cap].view(torch.float64)
 
 
 def workspace(nbytes, device):
@@ -96,6 +114,12 @@ class Ingress:
         if self.is_torch:
             return t.to(device=self.out_device, dtype=self.out_dtype)
         return t.detach().cpu().numpy().astype(self.out_dtype, copy=False)
+
+    def scalars(self, vals):
+        """List of scalars of the caller's kind, copied together."""
+        if self.is_torch and vals:
+            return list(torch.tensor(vals, dtype=self.out_dtype, device=self.out_device).unbind())
+        return [self.scalar(x) for x in vals]
 
     def scalar(self, val):
         """Scalar of the caller's kind (numpy scalar or 0-d tensor)."""

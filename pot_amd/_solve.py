@@ -24,9 +24,16 @@ class DenseResult:
     statuses: torch.Tensor = None  # (B,) int32 per-problem statuses (each=True only)
 
 
+def start(B, n, m, value, device):
+    """Constant starting potentials (B, n) and (B, m), from one fill."""
+    off = -(-B * n // 32) * 32
+    both = torch.full((off + B * m,), value, dtype=torch.float64, device=device)
+    return both[:B * n].view(B, n), both[off:].view(B, m)
+
+
 def dense_solve(M, a, b, u0, v0, reg, *, domain, order, kernel_given=False,
                 max_iter=1000, stop_thr=1e-9, err_norm=0, batch=None,
-                bstride=None, tile=None, each=False):
+                bstride=None, tile=None, each=False, own=False):
     """Run potamd_sinkhorn_dense (or, with ``each``, potamd_sinkhorn_dense_each:
     every problem stops on its own check, and the result's ``niters`` /
     ``statuses`` hold the per-problem stops).
@@ -34,6 +41,7 @@ def dense_solve(M, a, b, u0, v0, reg, *, domain, order, kernel_given=False,
     M: (n, m) or (B, n, m) device tensor (float32/float64), rows contiguous.
     a: (B, n), b: (B, m), u0: (B, n), v0: (B, m) float64 device tensors.
     ``batch``/``bstride`` override the batch layout (bstride = 0 shares M).
+    ``own``: u0 and v0 are float64, contiguous and the solver's to overwrite.
     """
     lib = _lib.load()
     dev = M.device
@@ -58,10 +66,13 @@ def dense_solve(M, a, b, u0, v0, reg, *, domain, order, kernel_given=False,
     if ws_bytes == 0:
         raise _lib.LibraryError("invalid shape for the dense solver")
     ws = _device.workspace(ws_bytes, dev)
-    u = u0.to(torch.float64).contiguous().clone()
-    v = v0.to(torch.float64).contiguous().clone()
+    if own:
+        u, v = u0, v0
+    else:
+        u = u0.to(torch.float64).contiguous().clone()
+        v = v0.to(torch.float64).contiguous().clone()
     err_cap = max(1, max_iter // 10 + 2)
-    err_hist = torch.zeros(err_cap, dtype=torch.float64, device=dev)
+    err_hist = _device.err_buffer(err_cap, dev)
     info = (ctypes.c_int * 4)()
     hc = _device.host_ctrl()
     if a.numel() != B * n or b.numel() != B * m or u.numel() != B * n or v.numel() != B * m:
@@ -91,7 +102,7 @@ def dense_solve(M, a, b, u0, v0, reg, *, domain, order, kernel_given=False,
             "a column mass fell below the fp32 range at iteration %d; "
             "use float64 inputs" % info[0])
     n_err = 0 if each else min(info[1], err_cap)
-    errs = err_hist[:n_err].cpu().tolist() if n_err else []
+    errs = err_hist[:n_err].tolist() if n_err else []
     return DenseResult(u=u.view(B, n), v=v.view(B, m), niter=info[0], errs=errs,
                        status=info[2], bad_iter=info[3], niters=niters, statuses=statuses)
 

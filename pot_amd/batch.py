@@ -112,11 +112,10 @@ def _projection(K, a, b, max_iter, tol, domain, grad):
     at = _weights_dev(a, ing, (B, n))
     bt = _weights_dev(b, ing, (B, m))
     init = 0.0 if domain == _lib.LOG else 1.0
-    u0 = torch.full((B, n), init, dtype=torch.float64, device=ing.device)
-    v0 = torch.full((B, m), init, dtype=torch.float64, device=ing.device)
+    u0, v0 = _solve.start(B, n, m, init, ing.device)
     res = _solve.dense_solve(Kt, at, bt, u0, v0, None, domain=domain,
                              order=_lib.ROW_FIRST, kernel_given=True,
-                             max_iter=max_iter, stop_thr=tol, err_norm=0)
+                             max_iter=max_iter, stop_thr=tol, err_norm=0, own=True)
     u, v = res.u, res.v
     if grad == "last_step":
         if requires_grad(K, a, b):
@@ -127,7 +126,7 @@ def _projection(K, a, b, max_iter, tol, domain, grad):
         # the same update on the device: one more row-first iteration
         res1 = _solve.dense_solve(Kt, at, bt, u, v, None, domain=domain,
                                   order=_lib.ROW_FIRST, kernel_given=True, max_iter=1,
-                                  stop_thr=0.0, err_norm=0)
+                                  stop_thr=0.0, err_norm=0, own=True)
         u, v = res1.u, res1.v
     P, L, _ = _solve.plan(Kt, u, v, None, domain=domain, kernel_given=True,
                           want_log=domain == _lib.LOG, want_sums=0)
@@ -336,10 +335,9 @@ def solve_batch(M, reg, a=None, b=None, max_iter=1000, tol=1e-5, solver="log_sin
     at = _weights_dev(a, ing, (B, n))
     bt = _weights_dev(b, ing, (B, m))
     init = 0.0 if domain == _lib.LOG else 1.0
-    u0 = torch.full((B, n), init, dtype=torch.float64, device=ing.device)
-    v0 = torch.full((B, m), init, dtype=torch.float64, device=ing.device)
+    u0, v0 = _solve.start(B, n, m, init, ing.device)
     res = _solve.dense_solve(Mt, at, bt, u0, v0, reg, domain=domain, order=_lib.ROW_FIRST,
-                             max_iter=max_iter, stop_thr=tol, err_norm=0)
+                             max_iter=max_iter, stop_thr=tol, err_norm=0, own=True)
     u, v = res.u, res.v
     log = {"n_iter": res.niter}
 
@@ -359,7 +357,7 @@ def solve_batch(M, reg, a=None, b=None, max_iter=1000, tol=1e-5, solver="log_sin
             return OTResult(value=value, value_linear=value_linear, potentials=(un, vn),
                             plan=T, log=log)
         res1 = _solve.dense_solve(Mt, at, bt, u, v, reg, domain=domain, order=_lib.ROW_FIRST,
-                                  max_iter=1, stop_thr=0.0, err_norm=0)
+                                  max_iter=1, stop_thr=0.0, err_norm=0, own=True)
         u, v = res1.u, res1.v
 
     P, _, sums = _solve.plan(Mt, u, v, reg, domain=domain, a=at, b=bt,

@@ -225,8 +225,7 @@ def sinkhorn_log(a, b, M, reg, numItermax=1000, stopThr=1e-9, verbose=False,
         return out
 
     if warmstart is None:
-        u0 = torch.zeros((1, n), dtype=torch.float64, device=ing.device)
-        v0 = torch.zeros((1, m), dtype=torch.float64, device=ing.device)
+        u0, v0 = _solve.start(1, n, m, 0.0, ing.device)
     else:
         u0 = ing.dev(warmstart[0], torch.float64).view(1, n)
         v0 = ing.dev(warmstart[1], torch.float64).view(1, m)
@@ -240,7 +239,7 @@ def sinkhorn_log(a, b, M, reg, numItermax=1000, stopThr=1e-9, verbose=False,
     else:
         res = _solve.dense_solve(Mt, at.view(1, n), bt.view(1, m), u0, v0, reg,
                                  domain=_lib.LOG, order=_lib.COL_FIRST,
-                                 max_iter=numItermax, stop_thr=stopThr)
+                                 max_iter=numItermax, stop_thr=stopThr, own=warmstart is None)
         u, v, errs, niter = res.u, res.v, res.errs, res.niter
         if verbose:
             _print_errs(errs)
@@ -256,7 +255,7 @@ def sinkhorn_log(a, b, M, reg, numItermax=1000, stopThr=1e-9, verbose=False,
         log_u = ing.out(u[0])
         log_v = ing.out(v[0])
         logd = {
-            "err": [ing.scalar(e) for e in errs],
+            "err": ing.scalars(errs),
             "niter": niter,
             "log_u": log_u,
             "log_v": log_v,
@@ -338,7 +337,8 @@ def sinkhorn_knopp(a, b, M, reg, numItermax=1000, stopThr=1e-9, verbose=False,
     else:
         res = _solve.dense_solve(Mt, a_b, b_b, u0, v0, reg, domain=_lib.SCALING,
                                  order=_lib.COL_FIRST, max_iter=numItermax,
-                                 stop_thr=stopThr, err_norm=1, batch=B, bstride=0)
+                                 stop_thr=stopThr, err_norm=1, batch=B, bstride=0,
+                                 own=warmstart is None)
         u, v, errs, niter = res.u, res.v, res.errs, res.niter
         if res.status == _lib.NUMERICAL:
             warnings.warn("Warning: numerical errors at iteration %d" % res.bad_iter)
@@ -364,7 +364,7 @@ def sinkhorn_knopp(a, b, M, reg, numItermax=1000, stopThr=1e-9, verbose=False,
     if log:
         uu = u.t() if nh else u[0]
         vv = v.t() if nh else v[0]
-        logd = {"err": [ing.scalar(e) for e in errs], "niter": niter,
+        logd = {"err": ing.scalars(errs), "niter": niter,
                 "u": ing.out(uu), "v": ing.out(vv)}
     if _grad_parts:
         return ing, sums[0, 0].item(), P[0], torch.log(u[0]), torch.log(v[0]), logd

@@ -117,7 +117,7 @@ def empirical_sinkhorn(X_s, X_t, reg, a=None, b=None, metric="sqeuclidean", numI
                               verbose, warn, warmstart)
         f_o, g_o = ing.out(f), ing.out(g)
         if log:
-            return f_o, g_o, {"err": [ing.scalar(e) for e in lg["err"]], "u": f_o, "v": g_o,
+            return f_o, g_o, {"err": ing.scalars(lg["err"]), "u": f_o, "v": g_o,
                               "niter": lg["niter"],
                               "lazy_plan": get_sinkhorn_lazytensor(X_s, X_t, f_o, g_o, metric,
                                                                    reg)}
@@ -148,7 +148,7 @@ def empirical_sinkhorn2(X_s, X_t, reg, a=None, b=None, metric="sqeuclidean",
         loss = ing.scalar(sums["cost"])
         if log:
             f_o, g_o = ing.out(f), ing.out(g)
-            return loss, {"err": [ing.scalar(e) for e in lg["err"]], "u": f_o, "v": g_o,
+            return loss, {"err": ing.scalars(lg["err"]), "u": f_o, "v": g_o,
                           "niter": lg["niter"],
                           "lazy_plan": get_sinkhorn_lazytensor(X_s, X_t, f_o, g_o, metric, reg)}
         return loss

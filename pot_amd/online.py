@@ -90,7 +90,7 @@ def sinkhorn_online(X, Y, reg, a=None, b=None, numItermax=1000, stopThr=1e-9, *,
         u = torch.as_tensor(warmstart[0]).to(device=dev, dtype=torch.float64).reshape(-1).clone()
     v = torch.zeros(m, dtype=torch.float64, device=dev)
     err_cap = max(1, numItermax // 10 + 2)
-    err_hist = torch.zeros(err_cap, dtype=torch.float64, device=dev)
+    err_hist = _device.err_buffer(err_cap, dev)
     info = (ctypes.c_int * 4)()
     scale_out = ctypes.c_double(0.0)
     hc = _device.host_ctrl()
@@ -108,7 +108,7 @@ def sinkhorn_online(X, Y, reg, a=None, b=None, numItermax=1000, stopThr=1e-9, *,
         warnings.warn("Sinkhorn did not converge. You might want to "
                       "increase the number of iterations `numItermax` "
                       "or the regularization parameter `reg`.")
-    out = {"niter": info[0], "err": err_hist[:n_err].cpu().tolist() if n_err else [],
+    out = {"niter": info[0], "err": err_hist[:n_err].tolist() if n_err else [],
            "status": rc, "cost_scale": scale_out.value, "precision": precision,
            "a": at, "b": bt}
     return u, v, out

@@ -37,8 +37,7 @@ raises when a gradient is needed.
 import numpy as np
 import torch
 
-from . import _solve
-from . import batch as _batch
+from . import _lib, _solve
 from ._device import require_gpu
 from ._grad import requires_grad
 from .utils import OTResult
@@ -274,14 +273,36 @@ def solve_gromov_batch(C1, C2, reg=1e-2, a=None, b=None, loss="sqeuclidean", sym
         T = T_init.detach()
     log_T = torch.log(T + EPS_LOG)
     proj, step = None, -1
+    h1, h2 = _as_channels(Ld["hC1"]), _as_channels(Ld["hC2"])
+    a64, b64 = ad.to(torch.float64).contiguous(), bd.to(torch.float64).contiguous()
     with torch.no_grad():
+        # log T - lin / reg, where lin = (1 - alpha) M + 2 alpha (constC - w S):
+        # the part that stays, then S added by the products themselves (the
+        # separable part of a product with zero marginals is not formed)
+        const = ((1 - alpha) * Md + (2 * alpha) * Ld["constC"]) / reg
+        w = 2.0 * float(alpha) * (1.0 if symmetric else 0.5)
+        many = isinstance(reg, torch.Tensor) and reg.numel() > 1  # a reg per problem
+        gain = w if many else w / float(reg) if reg else float("inf")
         for step in range(max_iter):
-            lin = (1 - alpha) * Md + (2 * alpha) * tensor_product_batch(Ld, T,
-                                                                         symmetric=symmetric)
-            proj = _batch.bregman_log_projection_batch(log_T - lin / reg, ad, bd,
-                                                       max_iter=max_iter_inner, tol=tol_inner)
-            change = torch.max(torch.mean(torch.abs(proj["T"] - T), dim=(1, 2)))
-            T, log_T = proj["T"], proj["log_T"]
+            T = T.contiguous()
+            K = log_T - const
+            S = torch.zeros_like(K) if many else K
+            for d in range(h1.shape[-1]):
+                h1d, h2d = h1[..., d], h2[..., d]
+                _solve.gemm(_solve.bmm(h1d, T), h2d, S, alpha=gain, beta=1.0, transB=True)
+                if not symmetric:
+                    _solve.gemm(_solve.bmm(h1d, T, transA=True), h2d, S, alpha=gain, beta=1.0)
+            if many:
+                K += S / reg
+            u0, v0 = _solve.start(B, n, m, 0.0, K.device)
+            res = _solve.dense_solve(K, a64, b64, u0, v0, None, domain=_lib.LOG,
+                                     order=_lib.ROW_FIRST, kernel_given=True,
+                                     max_iter=max_iter_inner, stop_thr=tol_inner, own=True)
+            P, log_T, _ = _solve.plan(K, res.u, res.v, None, domain=_lib.LOG, kernel_given=True,
+                                      want_log=True, want_sums=0)
+            proj = (res.u, res.v)
+            change = torch.linalg.vector_norm(P - T, ord=1, dim=(1, 2)).max().item() / (n * m)
+            T = P
             if change < tol:
                 break
 
@@ -293,7 +314,7 @@ def solve_gromov_batch(C1, C2, reg=1e-2, a=None, b=None, loss="sqeuclidean", sym
     value_quad = torch.sum(tensor_product_batch(L, T, recompute_const=True,
                                                 symmetric=symmetric) * T, dim=(1, 2))
     value = (1 - alpha) * value_linear + alpha * value_quad
-    potentials = None if proj is None else tuple(conv.out(x) for x in proj["potentials"])
+    potentials = None if proj is None else tuple(conv.out(x.to(C1.dtype)) for x in proj)
     return OTResult(value=conv.out(value), value_linear=conv.out(value_linear * (1 - alpha)),
                     value_quad=conv.out(value_quad * alpha), plan=conv.out(T),
                     potentials=potentials, log={"n_iter": step})

@@ -57,7 +57,7 @@ def _stabilized_device(ing, Mt, at, bt, reg, numItermax, tau, stopThr, warmstart
     u = torch.empty(n, dtype=torch.float64, device=dev)
     v = torch.empty(m, dtype=torch.float64, device=dev)
     err_cap = max(1, numItermax // print_period + 2)
-    err_hist = torch.zeros(err_cap, dtype=torch.float64, device=dev)
+    err_hist = _device.err_buffer(err_cap, dev)
     marg = torch.zeros(2, dtype=torch.float64, device=dev) if want_marg else None
     code = _lib.F32 if Mt.dtype == torch.float32 else _lib.F64
     ws_bytes = lib.potamd_stabilized_workspace_size(code, n, m)
@@ -75,7 +75,7 @@ def _stabilized_device(ing, Mt, at, bt, reg, numItermax, tau, stopThr, warmstart
     elif rc == _lib.MAX_ITER and warn:
         warnings.warn(NOT_CONVERGED)
     n_err = min(info[1], err_cap)
-    errs = err_hist[:n_err].cpu().tolist() if n_err else []
+    errs = err_hist[:n_err].tolist() if n_err else []
     return alpha, beta, u, v, errs, info[0], marg
 
 
@@ -96,7 +96,7 @@ def _stabilized_multi(ing, Mt, at, bt, reg, numItermax, tau, stopThr, warmstart,
     u = torch.empty((H, n), dtype=torch.float64, device=dev)
     v = torch.empty((H, m), dtype=torch.float64, device=dev)
     err_cap = max(1, numItermax // print_period + 2)
-    err_hist = torch.zeros(err_cap, dtype=torch.float64, device=dev)
+    err_hist = _device.err_buffer(err_cap, dev)
     code = _lib.F32 if Mt.dtype == torch.float32 else _lib.F64
     ws_bytes = lib.potamd_stabilized_multi_workspace_size(code, n, m, H)
     ws = _device.workspace(ws_bytes, dev)
@@ -113,7 +113,7 @@ def _stabilized_multi(ing, Mt, at, bt, reg, numItermax, tau, stopThr, warmstart,
     elif rc == _lib.MAX_ITER and warn:
         warnings.warn(NOT_CONVERGED)
     n_err = min(info[1], err_cap)
-    errs = err_hist[:n_err].cpu().tolist() if n_err else []
+    errs = err_hist[:n_err].tolist() if n_err else []
     if verbose:
         _print_checks(errs, print_period)
     logu = alpha[None, :] / reg + torch.log(u)  # (H, n)
@@ -125,7 +125,7 @@ def _stabilized_multi(ing, Mt, at, bt, reg, numItermax, tau, stopThr, warmstart,
         return out
     al = alpha[:, None] + reg * torch.log(u.t())
     be = beta[:, None] + reg * torch.log(v.t())
-    logd = {"err": [ing.scalar(e) for e in errs], "n_iter": info[0], "logu": ing.out(logu.t()),
+    logd = {"err": ing.scalars(errs), "n_iter": info[0], "logu": ing.out(logu.t()),
             "logv": ing.out(logv.t()), "alpha": ing.out(al), "beta": ing.out(be)}
     logd["warmstart"] = (logd["alpha"], logd["beta"])
     return out, logd
@@ -155,7 +155,7 @@ def sinkhorn_stabilized(a, b, M, reg, numItermax=1000, tau=1e3, stopThr=1e-9, wa
     if log:
         al = alpha + reg * torch.log(u)
         be = beta + reg * torch.log(v)
-        logd = {"err": [ing.scalar(e) for e in errs], "n_iter": niter, "logu": ing.out(logu),
+        logd = {"err": ing.scalars(errs), "n_iter": niter, "logu": ing.out(logu),
                 "logv": ing.out(logv), "alpha": ing.out(al), "beta": ing.out(be)}
         logd["warmstart"] = (logd["alpha"], logd["beta"])
         return out, logd
@@ -213,7 +213,7 @@ def sinkhorn_epsilon_scaling(a, b, M, reg, numItermax=100, epsilon0=1e4, numInne
                           want_sums=0)
     G = ing.out(P[0])
     if log:
-        logd = {"err": [ing.scalar(e) for e in errs], "alpha": ing.out(alpha),
+        logd = {"err": ing.scalars(errs), "alpha": ing.out(alpha),
                 "beta": ing.out(beta), "niter": ii}
         logd["warmstart"] = (logd["alpha"], logd["beta"])
         return G, logd
