@@ -142,8 +142,9 @@ struct Words {
 Words words_of(int B, int n, int m, const Choice& c) {
   const int rbs = (n + c.R - 1) / c.R, cbs = (m + c.C - 1) / c.C;
   Words w;
-  w.row_slot = c.C > 1 ? (int64_t)(rbs + 1) * c.C * 2 : 0;  // (and a flag)
-  w.col_slot = c.R > 1 ? (int64_t)(cbs + 1) * c.R * 2 : 0;
+  // Each member's values (and a flag), and the totals.
+  w.row_slot = c.C > 1 ? (int64_t)(rbs + 1) * (c.C + 1) * 2 : 0;
+  w.col_slot = c.R > 1 ? (int64_t)(cbs + 1) * (c.R + 1) * 2 : 0;
   w.err_slot = (int64_t)B * std::max(c.R, c.C) * 2;
   w.col_base = (int64_t)B * c.R * 2 * w.row_slot;
   w.err_base = w.col_base + (int64_t)B * c.C * 2 * w.col_slot;

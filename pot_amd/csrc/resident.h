@@ -222,17 +222,19 @@ __global__ __launch_bounds__(64 * W) void resident_kernel(ResidentArgs A) {
   word_t* const xcol = A.words + A.col_base + (int64_t)(p * GC + J) * 2 * A.col_slot;
   word_t* const xerr = A.words + A.err_base;
 
-  // Reads N = G x L tagged values into LDS; value w, entry w % L of member
-  // w / L, lands at (w % L) * GS + w / L.  A lane reads 16 bytes, two tagged words (one double
-  // or two floats), past the caches that are not coherent.
-  auto gather = [&](auto* dst, word_t* src, int N, int L, int GS, unsigned tag) {
-    using P = typename std::remove_pointer<decltype(dst)>::type;
-    constexpr int PER = 2 / (sizeof(P) / 4);  // values a read
-    constexpr int Q = 4;
-    const int units = (N + PER - 1) / PER;
-    const rsrc_t rsrc = slot_at(src, units * 2);
+  // Polls units tagged entries of BYTES each until all carry the tag: entry w
+  // lies at byte at(w) of the slot, and take(w, entry) keeps a complete one.
+  // Entries are read past the caches that are not coherent.  `pause`: 512
+  // clocks first: the entries of members that left the last
+  // exchange with this one are then there at the first read, which otherwise
+  // comes back too early and costs a second one (2048^2 float64 8.0 -> 7.0 us
+  // an iteration; single float words arrive sooner and do without).
+  auto poll = [&](auto bytes, rsrc_t rsrc, int units, bool pause, unsigned tag, auto at, auto take) {
+    constexpr int Q = ER == 10 ? 5 : 4;  // reads of a thread in flight
+    using V = typename std::conditional<decltype(bytes)::value == 16, u32x4, u32x2>::type;
+    if (pause) __builtin_amdgcn_s_sleep(8);
     for (int w0 = tid; w0 < units; w0 += Q * T) {
-      u32x4 v[Q];
+      V v[Q];
       unsigned pend = 0;
 #pragma unroll
       for (int q = 0; q < Q; ++q) pend |= (w0 + q * T < units ? 1u : 0u) << q;
@@ -241,24 +243,15 @@ __global__ __launch_bounds__(64 * W) void resident_kernel(ResidentArgs A) {
         asm volatile("" ::: "memory");  // read anew each time
 #pragma unroll
         for (int q = 0; q < Q; ++q)
-          if (pend >> q & 1)
-            v[q] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (w0 + q * T) * 16, 0, kAgent);
-#pragma unroll
-        for (int q = 0; q < Q; ++q) {
-          if (!(pend >> q & 1)) continue;
-          const int w = (w0 + q * T) * PER;
-          const bool second = sizeof(P) == 8 || w + 1 < N;
-          if (v[q][1] == tag && (!second || v[q][3] == tag)) {
-            if constexpr (sizeof(P) == 8) {
-              dst[(w % L) * GS + w / L] =
-                  __longlong_as_double((long long)(((word_t)v[q][2] << 32) | v[q][0]));
-            } else {
-              dst[(w % L) * GS + w / L] = __uint_as_float(v[q][0]);
-              if (second) dst[((w + 1) % L) * GS + (w + 1) / L] = __uint_as_float(v[q][2]);
-            }
-            pend &= ~(1u << q);
+          if (pend >> q & 1) {
+            if constexpr (sizeof(V) == 16)
+              v[q] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, at(w0 + q * T), 0, kAgent);
+            else
+              v[q] = __builtin_amdgcn_raw_buffer_load_b64(rsrc, at(w0 + q * T), 0, kAgent);
           }
-        }
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+          if (pend >> q & 1 && take(w0 + q * T, v[q])) pend &= ~(1u << q);
         if (pend) {
           __builtin_amdgcn_s_sleep(1);
           if ((spin & 63) == 63) {
@@ -274,13 +267,41 @@ __global__ __launch_bounds__(64 * W) void resident_kernel(ResidentArgs A) {
       }
     }
   };
+  using Bytes8 = std::integral_constant<int, 8>;
+  using Bytes16 = std::integral_constant<int, 16>;
+  auto as_double = [](u32x4 v) {
+    return __longlong_as_double((long long)(((word_t)v[2] << 32) | v[0]));
+  };
+  // Reads N = G x L tagged values into LDS; value w, entry w % L of member
+  // w / L, lands at (w % L) * GS + w / L.  A lane reads 16 bytes, two tagged
+  // words (one double or two floats).
+  auto gather = [&](auto* dst, word_t* src, int N, int L, int GS, unsigned tag) {
+    using P = typename std::remove_pointer<decltype(dst)>::type;
+    constexpr int PER = 2 / (sizeof(P) / 4);  // values a read
+    const int units = (N + PER - 1) / PER;
+    poll(Bytes16(), slot_at(src, units * 2), units, sizeof(P) == 8 || units > T, tag,
+         [&](int w) { return w * 16; },
+         [&](int u, u32x4 v) {
+           const int w = u * PER;
+           const bool second = sizeof(P) == 8 || w + 1 < N;
+           if (v[1] != tag || (second && v[3] != tag)) return false;
+           if constexpr (sizeof(P) == 8) {
+             dst[(w % L) * GS + w / L] = as_double(v);
+           } else {
+             dst[(w % L) * GS + w / L] = __uint_as_float(v[0]);
+             if (second) dst[((w + 1) % L) * GS + (w + 1) / L] = __uint_as_float(v[2]);
+           }
+           return true;
+         });
+  };
   // Sum or maximum of x over the G members of this block's row or column
   // group, for the owner of entry idx < L; every thread takes part.
   // (Stabilised: with one more entry, the member's flag; `raised` says whether
   // one of the members did.)
   bool raised = false;
+  constexpr bool TWO = BLK && !STAB && ER * EC >= 64;  // (smaller blocks have fewer values)
   auto exchange = [&](auto x, bool own, int idx, int L, int G, int me, word_t* slots, int slot,
-                      unsigned& tag, auto maxop, bool flag) -> double {
+                      int room, unsigned& tag, auto maxop, bool flag) -> double {
     if (STAB) ++L;
     using P = decltype(x);
     constexpr bool MAX = decltype(maxop)::value;
@@ -290,6 +311,43 @@ __global__ __launch_bounds__(64 * W) void resident_kernel(ResidentArgs A) {
     if (STAB && tid == 0) value_put(slot_at(base, slot), me * L + L - 1, (P)(flag ? 1 : 0), tag);
     P* dst = reinterpret_cast<P*>(xs);
     const int GS = G | 1;
+    if constexpr (TWO) if (G * L * (int)sizeof(P) > 64 * T) {
+      // Many values: each member reads and adds a G-th of the entries and the
+      // totals are exchanged again: two waits of a read or two a thread in
+      // place of one of more than eight (all members read all G x L values).
+      // 2800^2 float64 (22 members, 255 rows) 11.7 -> 8.1 us an iteration;
+      // 5000 x 800 (20 members, 115 columns) 8.8 this way and 7.8 the other.
+      const int S = (L + G - 1) / G, s0 = min(me * S, L), cnt = min(S, L - s0);
+      constexpr int VB = 2 * sizeof(P);
+      poll(std::integral_constant<int, VB>(), slot_at(base, slot), G * cnt, sizeof(P) == 8, tag,
+           [&](int w) { return (w / cnt * L + s0 + w % cnt) * VB; },
+           [&](int w, auto v) {
+             bool all = v[1] == tag;
+             if constexpr (VB == 16) all = all && v[3] == tag;
+             if (!all) return false;
+             if constexpr (VB == 16)
+               dst[w % cnt * GS + w / cnt] = as_double(v);
+             else
+               dst[w % cnt * GS + w / cnt] = __uint_as_float(v[0]);
+             return true;
+           });
+      __syncthreads();
+      const rsrc_t totals = slot_at(base + slot - 2 * room, 2 * room);
+      if (tid < cnt) {
+        double s = (double)dst[tid * GS];
+        for (int k = 1; k < G; ++k) s = op2<MAX>(s, (double)dst[tid * GS + k]);
+        value_put(totals, s0 + tid, s, tag);
+      }
+      double* tot = xs + (S * GS * sizeof(P) + 7) / 8;
+      poll(Bytes16(), totals, L, true, tag, [&](int w) { return w * 16; },
+           [&](int w, u32x4 v) {
+             if (v[1] != tag || v[3] != tag) return false;
+             tot[w] = as_double(v);
+             return true;
+           });
+      __syncthreads();
+      return own ? tot[idx] : 0.0;
+    }
     gather(dst, base, L * G, L, GS, tag);
     __syncthreads();
     if (STAB) raised = __any(lane < G && dst[(L - 1) * GS + lane] != (P)0);
@@ -303,10 +361,10 @@ __global__ __launch_bounds__(64 * W) void resident_kernel(ResidentArgs A) {
   using Sum = std::false_type;
   using Max = std::true_type;
   auto rows_of = [&](auto x, auto maxop, bool flag = false) -> double {  // row owners
-    return exchange(x, rown, rl, nr, GC, J, xrow, A.row_slot, tag_r, maxop, flag);
+    return exchange(x, rown, rl, nr, GC, J, xrow, A.row_slot, A.rbs + 1, tag_r, maxop, flag);
   };
   auto cols_of = [&](auto x, auto maxop, bool flag = false) -> double {  // column owners
-    return exchange(x, cown, tid, nc, GR, I, xcol, A.col_slot, tag_c, maxop, flag);
+    return exchange(x, cown, tid, nc, GR, I, xcol, A.col_slot, A.cbs + 1, tag_c, maxop, flag);
   };
   auto abandon = [&]() {
     if (tid == 0) {

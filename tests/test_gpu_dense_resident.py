@@ -203,3 +203,24 @@ def test_stabilized_absorbs_as_the_oracle(n, m, tau, iters, dtype):
         assert np.max(np.abs(lg[key].double().cpu().numpy() - log[key])) < tol
     np.testing.assert_allclose([float(e) for e in lg["err"]], log["err"], rtol=max(tol, 1e-6),
                                atol=1e-12 if dtype == F64 else 1e-7)
+
+
+@pytest.mark.parametrize("n,m,dtype", [(9000, 128, F64), (250, 8190, F64), (9000, 250, F32),
+                                       (2801, 2790, F64)])
+def test_many_values_to_exchange(n, m, dtype):
+    """Column or row groups of so many values that their members add a part
+    each and exchange the totals."""
+    M, a, b = _problem(1, n, m, dtype, n + m)
+    reg = 0.05
+    for domain in (_lib.LOG, _lib.SCALING):
+        fn = osk.sinkhorn_log if domain == _lib.LOG else osk.sinkhorn_knopp
+        P, log = fn(a[0], b[0], M[0].astype(np.float64), reg, numItermax=12, stopThr=0.0, log=True,
+                    warn=False)
+        r = _solve_gpu(M, a, b, reg, domain, _lib.COL_FIRST, max_iter=12, stop_thr=0.0,
+                       err_norm=domain)
+        np.testing.assert_allclose(r.errs, log["err"], rtol=1e-9 if dtype == F64 else 1e-2,
+                                   atol=1e-9 if dtype == F64 else 1e-6)
+        u, v = r.u[0].cpu().numpy(), r.v[0].cpu().numpy()
+        if domain == _lib.SCALING:
+            u, v = np.log(u), np.log(v)
+        _check_plan(M[0], reg, u, v, P, dtype)
