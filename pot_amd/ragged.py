@@ -392,6 +392,63 @@ def split_plan(ns, ms, cus=None, regs=None):
     return parts
 
 
+# Size tiers of the automatic split: the least elements for 2, 4 and 8 parts.
+_NEVER = 1 << 62
+_TIERS = ((_NEVER, _NEVER, _NEVER), (1 << 17, _NEVER, _NEVER), (1 << 16, _NEVER, _NEVER),
+          (1 << 17, 3 << 17, _NEVER), (1 << 16, 1 << 17, _NEVER), (1 << 17, 3 << 17, 3 << 18),
+          (1 << 16, 1 << 17, 3 << 17))
+# A problem's fixed microseconds an iteration by parts (column reductions,
+# updates, the exchange), at 4 column tiles a wave.
+_FIXED_US = {1: 6.9, 2: 8.2, 4: 8.4, 8: 10.0}
+
+
+def auto_plan(ns, ms, cus=None):
+    """Workgroups per problem of the automatic split: the size tiers that make
+    the time of the GPU's work or of the longest problem, whichever is larger,
+    and half the other least.
+
+    The work is the parts' microseconds an iteration over the CUs.  The longest
+    problem is the slowest one's iteration times 0.35 sqrt(B): over batches of
+    Gaussian clouds the most iterations were 4 (40 problems) to 24 (3000) times
+    their mean, and which problem needs them is not known, so problems of one
+    size are split alike.  (A budget of one part a CU left the chip waiting for
+    unsplit problems.)  Milliseconds unsplit / with that budget / now: 512
+    problems of 64 to 1024 points 10.4 / 5.5 / 4.9, 300 of 200 to 900 16.8 / 17.1 /
+    9.9, 100 of 64 to 1024 5.1 / 2.4 / 2.0; 256 of 1024 points 18.3 / 18.8 / 7.5,
+    512 14.4 / 14.8 / 6.1, 2000 33.2 / - / 19.5.  Past 12 problems a CU the work
+    dominates (4096 of 1024 points: 30 to 53 unsplit, 36 in two parts).
+
+    The parts of a problem follow each other in the queue, so a part waits at
+    most for workgroups on earlier problems, whose parts are all taken."""
+    ns = np.asarray(ns, dtype=np.int64)
+    ms = np.asarray(ms, dtype=np.int64)
+    nm = ns * ms
+    one = np.ones(len(ns), dtype=np.int32)
+    if cus is None:
+        cus = torch.cuda.get_device_properties(_device.require_gpu()).multi_processor_count
+    if len(ns) == 0 or len(ns) > 12 * cus or nm.max() < 1 << 16:
+        return one
+    blocks = -(-ns // 32)
+    tiles = -(-ms // 256)                         # column tiles of a wave
+    wide = np.where(tiles <= 2, 2, 4)             # ... of a split problem's
+    t = {1: blocks * (0.15 + 0.25 * tiles) + _FIXED_US[1] * (0.5 + 0.125 * tiles)}
+    for k in (2, 4, 8):
+        t[k] = -(-blocks // k) * (0.15 + 0.25 * wide) + _FIXED_US[k] * (0.5 + 0.125 * wide)
+    best, spread = None, 0.35 * float(np.sqrt(len(ns)))
+    for two, four, eight in _TIERS:
+        parts, us = one, t[1]
+        for k, least in ((2, two), (4, four), (SPLIT_MAX, eight)):
+            if least == _NEVER:
+                continue
+            up = (nm >= least) & (ns >= 32 * k)
+            parts, us = np.where(up, np.int32(k), parts), np.where(up, t[k], us)
+        work, longest = float((us * parts).sum()) / cus, spread * float(us.max())
+        cost = max(work, longest) + 0.5 * min(work, longest)
+        if best is None or cost < best[0]:
+            best = cost, parts
+    return best[1]
+
+
 def _split_tables(parts):
     """split[p] = parts | slot << 4 for the split problems (0 otherwise) and
     the number of slots."""
@@ -527,8 +584,8 @@ def sinkhorn_log_ragged_points(P, u0=None, numItermax=1000, stopThr=1e-9, order=
     sweep and never stored.  ``cmax``: the maxima from ``points_cmax`` (the
     solve then skips its own search).  ``waves``: wavefronts per problem (8
     or 16; 0 = the autotuned value of this batch class, else the library
-    default).  ``split``: "auto" (``split_plan``: only batches too small to
-    fill the GPU are split), None (one workgroup per problem) or workgroups
+    default).  ``split``: "auto" (``auto_plan``: large problems of
+    batches whose longest would outlast the rest), None (one workgroup per problem) or workgroups
     per problem (1..8): a split problem's rows are shared by several
     workgroups (8 waves each).  ``unsolved``: "dense" (default) solves the
     problems the kernel cannot take (status 2: scaled coordinates outside its
@@ -568,7 +625,7 @@ def sinkhorn_log_ragged_points(P, u0=None, numItermax=1000, stopThr=1e-9, order=
         # (sizes only, as RaggedGraph plans before it sees the regs, so the
         # eager solve and a graph replay of one batch split alike and agree
         # bit for bit)
-        parts = split_plan(P.ns, P.ms) if (isinstance(split, str) and split == "auto") \
+        parts = auto_plan(P.ns, P.ms) if (isinstance(split, str) and split == "auto") \
             else _check_parts(split, P.ns)
     if parts is not None and (parts > 1).any():
         table, nsplit = _split_tables(parts)
@@ -645,7 +702,7 @@ class RaggedGraph:
         # the queue items re-ordered on each solve, the exchange slots zero.
         self.parts = None
         if split is not None and cost == "points":
-            parts = split_plan(self.ns, self.ms) if (isinstance(split, str) and split == "auto") \
+            parts = auto_plan(self.ns, self.ms) if (isinstance(split, str) and split == "auto") \
                 else _check_parts(split, self.ns)
             if (parts > 1).any():
                 self.parts = parts

@@ -244,3 +244,27 @@ def test_bregman_namespace_has_the_path_functions():
         assert callable(getattr(b, name)), name
     with pytest.raises(ValueError):
         b.sinkhorn([0.5, 0.5], [0.5, 0.5], [[0.0, 1.0], [1.0, 0.0]], 1.0, method="unknown")
+
+
+def test_auto_plan():
+    import numpy as np
+
+    from pot_amd import ragged
+    big, mid = np.full(64, 1024), np.full(64, 200)
+    # problems of one size are split alike; small ones and full batches are not
+    for B in (1, 40, 300, 2000):
+        parts = ragged.auto_plan(np.full(B, 1024), np.full(B, 1024), cus=256)
+        assert (parts == parts[0]).all() and parts[0] in (2, 4, 8), B
+    assert (ragged.auto_plan(mid, mid, cus=256) == 1).all()
+    assert (ragged.auto_plan(np.full(4096, 1024), np.full(4096, 1024), cus=256) == 1).all()
+    assert (ragged.auto_plan(np.full(49, 1024), np.full(49, 1024), cus=4) == 1).all()
+    assert len(ragged.auto_plan([], [], cus=256)) == 0
+    # every part has rows (32 a part), and larger problems no fewer parts
+    rng = np.random.default_rng(0)
+    ns, ms = rng.integers(32, 1025, 400), rng.integers(32, 1025, 400)
+    parts = ragged.auto_plan(ns, ms, cus=256)
+    assert (ns >= 32 * parts).all()
+    assert set(parts) <= {1, 2, 4, 8} and parts.max() > 1
+    ragged._check_parts(parts, ns)
+    mixed = ragged.auto_plan(np.concatenate([big, mid]), np.concatenate([big, mid]), cus=256)
+    assert mixed[:64].min() > 1 and (mixed[64:] == 1).all()
