@@ -415,8 +415,9 @@ def auto_plan(ns, ms, cus=None):
     unsplit problems.)  Milliseconds unsplit / with that budget / now: 512
     problems of 64 to 1024 points 10.4 / 5.5 / 4.9, 300 of 200 to 900 16.8 / 17.1 /
     9.9, 100 of 64 to 1024 5.1 / 2.4 / 2.0; 256 of 1024 points 18.3 / 18.8 / 7.5,
-    512 14.4 / 14.8 / 6.1, 2000 33.2 / - / 19.5.  Past 12 problems a CU the work
-    dominates (4096 of 1024 points: 30 to 53 unsplit, 36 in two parts).
+    512 14.4 / 14.8 / 6.1, 2000 33.2 / - / 19.5.  Past 8 problems a CU the work of
+    two parts is as long as most batches' longest problem (3000 of 1024 points: 23
+    and up unsplit, 27 in two parts; 4096: 30 to 53, 36).
 
     The parts of a problem follow each other in the queue, so a part waits at
     most for workgroups on earlier problems, whose parts are all taken."""
@@ -426,7 +427,7 @@ def auto_plan(ns, ms, cus=None):
     one = np.ones(len(ns), dtype=np.int32)
     if cus is None:
         cus = torch.cuda.get_device_properties(_device.require_gpu()).multi_processor_count
-    if len(ns) == 0 or len(ns) > 12 * cus or nm.max() < 1 << 16:
+    if len(ns) == 0 or len(ns) > 8 * cus or nm.max() < 1 << 16:
         return one
     blocks = -(-ns // 32)
     tiles = -(-ms // 256)                         # column tiles of a wave

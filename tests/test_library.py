@@ -257,7 +257,7 @@ def test_auto_plan():
         assert (parts == parts[0]).all() and parts[0] in (2, 4, 8), B
     assert (ragged.auto_plan(mid, mid, cus=256) == 1).all()
     assert (ragged.auto_plan(np.full(4096, 1024), np.full(4096, 1024), cus=256) == 1).all()
-    assert (ragged.auto_plan(np.full(49, 1024), np.full(49, 1024), cus=4) == 1).all()
+    assert (ragged.auto_plan(np.full(33, 1024), np.full(33, 1024), cus=4) == 1).all()
     assert len(ragged.auto_plan([], [], cus=256)) == 0
     # every part has rows (32 a part), and larger problems no fewer parts
     rng = np.random.default_rng(0)
