@@ -1,6 +1,9 @@
 // Host side of the register-resident dense solve (resident.h): choice of the
 // tile, the exchange workspace, and the launches.
+#include <string.h>
+
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <mutex>
 
@@ -232,10 +235,27 @@ int resident_solve(int dtype, ResidentArgs a, double* u_keep, double* v_keep, Ct
     a.segment = 0;
     a.resume = 0;
     a.it0 = 0;
+    // The kernel writes its outcome where the host reads it (a copy of it was a
+    // launch and its wait: 100 x 120 float64 CTRLFIG us a call), but for a
+    // batch whose problems all add to it.
+    a.host = nullptr;
+    void* seen = nullptr;
+    if (host_ctrl && !(a.each && a.B > 1)) {
+      if (hipHostGetDevicePointer(&seen, host_ctrl, 0) == hipSuccess)
+        a.host = static_cast<Ctrl*>(seen);
+      else
+        (void)hipGetLastError();
+    }
+    if (a.host) {
+      memset(hc, 0, sizeof(Ctrl));
+      std::atomic_thread_fence(std::memory_order_seq_cst);
+    }
     if (launch(a, nullptr) != hipSuccess) return -1;
-    if (hipMemcpyAsync(hc, a.ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, s) != hipSuccess ||
+    if ((!a.host &&
+         hipMemcpyAsync(hc, a.ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, s) != hipSuccess) ||
         hipStreamSynchronize(s) != hipSuccess)
       return -1;
+    if (a.host && !hc->done) hc->counter = 1;
   } else {
     // One launch per check interval; the state travels in u and v themselves
     // (base 2), and at most two intervals are queued past an unread decision.

@@ -78,7 +78,8 @@ struct ResidentArgs {
   unsigned long long* words;  // exchange slots
   int row_slot, col_slot;
   int64_t err_slot, col_base, err_base;
-  Ctrl* ctrl;            // counter != 0: abandoned
+  Ctrl* ctrl;
+  Ctrl* host;  // pinned, device-visible: the outcome (or null: it is in ctrl)            // counter != 0: abandoned
   // stabilised: u_in / v_in hold alpha / beta
   int stab, period;
   double reg, inv_reg, tau, u_start, v_start;

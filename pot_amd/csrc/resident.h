@@ -369,6 +369,7 @@ __global__ __launch_bounds__(64 * W) void resident_kernel(ResidentArgs A) {
   auto abandon = [&]() {
     if (tid == 0) {
       __hip_atomic_store(&A.ctrl->counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (A.host) A.host->counter = 1;
       if (A.segment) A.ctrl->done = 1;
     }
   };
@@ -849,7 +850,7 @@ __global__ __launch_bounds__(64 * W) void resident_kernel(ResidentArgs A) {
       A.niters[p] = niter;
       A.statuses[p] = status;
     }
-    Ctrl* q = A.ctrl;
+    Ctrl* q = A.host ? A.host : A.ctrl;
     if (gridDim.x == 1) q->counter = 0;  // no launch has cleared it
     if (A.each && A.B > 1) {
       atomicMax(&q->niter, niter);  // the last problem's stop
