@@ -219,20 +219,28 @@ struct OnlineMergeArgs {
   Ctrl* ctrl;
 };
 
-// New potential and shift of R point r from its S split partials, read by
-// `get`; returns its error term on a check.
+// Log-sum-exp (base 2) of partials: 2^mx acc (mx = -inf: acc is 0, or a NaN).
+struct Lse {
+  double mx, acc;
+};
 template <typename Get>
-__device__ __forceinline__ double merge_row(const OnlineMergeArgs& A, int r, int S, Get get) {
-  double mx = -__builtin_inf();
+__device__ __forceinline__ Lse lse_of(int s0, int s1, Get get) {
+  Lse x = {-__builtin_inf(), 0.0};
 #pragma unroll 8
-  for (int s = 0; s < S; ++s) mx = fmax(mx, get(s));
-  double I = -__builtin_inf();
-  if (mx > -__builtin_inf()) {
-    double acc = 0.0;
+  for (int s = s0; s < s1; ++s) x.mx = fmax(x.mx, get(s));
+  if (x.mx > -__builtin_inf()) {
 #pragma unroll 8
-    for (int s = 0; s < S; ++s) acc += exp2(get(s) - mx);
-    I = mx + log2(acc);
+    for (int s = s0; s < s1; ++s) x.acc += exp2(get(s) - x.mx);
+  } else {
+    for (int s = s0; s < s1; ++s) x.acc = get(s) != get(s) ? __builtin_nan("") : x.acc;
   }
+  return x;
+}
+
+// New potential and shift of R point r from its partials; returns its error
+// term on a check.
+__device__ __forceinline__ double merge_row(const OnlineMergeArgs& A, int r, Lse x) {
+  const double I = x.mx > -__builtin_inf() ? x.mx + log2(x.acc) : -__builtin_inf();
   const double s2 = s2_of(A.cscale, A.reg);
   const double L2 = I - s2 * A.norm[r];
   const double wr = A.w[r];
@@ -295,7 +303,7 @@ __device__ __forceinline__ void mma_chunk(f32x16& acc, u32x4 a, u32x4 b) {
 // error of x . y is a third (rms 6e-8 of its mean size at d = 64, against
 // 1.8e-7: 9 roundings of full size for 32).  16384^2 points, d = 64: 201 us a
 // pass, 313 before; matrix cores 46% busy, VALU 37%.  d <= 16 takes one K step
-// of 16 instead of two: 5000 x 4000 points in 3-D, 14.4 us a pass, 22 before.
+// of 16 instead of two: 5000 x 4000 points in 3-D, 14.9 us a pass, 22 before.
 template <int P, int D, int MODE>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(
     ((P == POTAMD_ONLINE_BF16X3 && D == 64) || (P == POTAMD_ONLINE_F32 && D <= 64)) && MODE == kModeLse
@@ -605,14 +613,32 @@ void online_pass_kernel(PassArgs A) {
                                     __HIP_MEMORY_SCOPE_AGENT) == S - 1;
     __syncthreads();
     if (!last) return;
+    // Two threads a row, half of the splits each (one took 2.4 us of a pass at
+    // 16 splits; 5000 x 4000 points in 3-D 15.5 us a pass, 14.9 so).
     double e2 = 0.0;
-    const int row = blockIdx.x * kRowsPerWG + tid;
-    if (tid < kRowsPerWG && row < A.nr) {
+    Lse* halves = reinterpret_cast<Lse*>(sm_t[0][0]);  // (the tiles are done)
+    static_assert(T == 2 * kRowsPerWG && TILE >= kRowsPerWG * (int)sizeof(Lse), "two threads a row");
+    const int lrow = tid & (kRowsPerWG - 1), row = blockIdx.x * kRowsPerWG + lrow;
+    const int mid = (S + 1) / 2, s0 = tid < kRowsPerWG ? 0 : mid, s1 = tid < kRowsPerWG ? mid : S;
+    Lse x = {-__builtin_inf(), 0.0};
+    if (row < A.nr) {
       const double* pr = A.part + row;
-      e2 = merge_row(A.merge, row, S, [&](int s) {
+      x = lse_of(s0, s1, [&](int s) {
         return __hip_atomic_load(pr + (int64_t)s * A.nr_pad, __ATOMIC_RELAXED,
                                  __HIP_MEMORY_SCOPE_AGENT);
       });
+    }
+    if (tid >= kRowsPerWG) halves[lrow] = x;
+    __syncthreads();
+    if (tid < kRowsPerWG && row < A.nr) {
+      const Lse y = halves[lrow];
+      if (y.mx > x.mx) {
+        x.acc = (x.mx > -__builtin_inf() ? x.acc * exp2(x.mx - y.mx) : x.acc) + y.acc;
+        x.mx = y.mx;
+      } else {
+        x.acc += y.mx > -__builtin_inf() ? y.acc * exp2(y.mx - x.mx) : y.acc;
+      }
+      e2 = merge_row(A.merge, row, x);
     }
     if (tid == 0) A.tickets[blockIdx.x] = 0;  // for the next pass
     if (A.merge.check && tid < kRowsPerWG) {
@@ -826,7 +852,7 @@ __global__ __launch_bounds__(kMergeRows) void online_merge_kernel(OnlineMergeArg
   double e2 = 0.0;
   if (r < A.nr) {
     const double* pr = A.part + r;
-    e2 = merge_row(A, r, A.S, [&](int s) { return pr[(int64_t)s * A.nr_pad]; });
+    e2 = merge_row(A, r, lse_of(0, A.S, [&](int s) { return pr[(int64_t)s * A.nr_pad]; }));
   }
   if (!A.check) return;
   e2 = wave_sum(e2);
@@ -1202,7 +1228,15 @@ hipError_t half_step(int prec, int D, int d, const Side& R, const Side& C, const
                      const OnlineLayout& L, double reg, int S, OnlineMergeArgs& ma,
                      hipStream_t s) {
   const int nsteps = (C.count + kStep - 1) / kStep;
-  const int sps = (nsteps + S - 1) / S;
+  int sps = (nsteps + S - 1) / S;
+  // Whole stages (a part of one costs as much as all of it: 5000 x 4000 points
+  // in 3-D, 13 splits of two and a half stages of 128 16.6 us a pass, 16 of two
+  // 15.5), fewer a split while their partials have room.
+  const int stage = prec == POTAMD_ONLINE_F64 ? 1 : stage_points(prec, D) / kStep;
+  if (stage > 1 && sps % stage) {
+    sps -= sps % stage;
+    if (sps == 0 || (nsteps + sps - 1) / sps > 64) sps += stage;
+  }
   const int Seff = (nsteps + sps - 1) / sps;
   ma.part = L.part;
   ma.S = Seff;
