@@ -113,7 +113,14 @@ struct Choice {
 // float64; blocked 4.9 us at 300^2 (3 x 3), 6.3 at 1000 x 900, 7.5 at 2048^2
 // (16 x 16); the row sweep took 12, 12, 12, 13, 25 and 37 us).  So a problem
 // that fits one workgroup stays in one.
-Choice choose(int dtype, int B, int n, int m) {
+// Of two tiles of one size (128 x 128 by eight waves or by four of twice the
+// elements) the fewer waves where there are more problems than CUs, as more such
+// workgroups are resident at once (300 problems of 110 x 90 7.2 us an iteration
+// in segments, 2.5 so; float32 5.5, 1.8), and for a float64 problem in the log
+// domain, whose waves each have their own checks (64 of 100^2 1.88, 1.73; the
+// scaling domain 1.41, 1.48; float32 1.31, 1.41).  Both have the same exchange
+// words.
+Choice choose(int dtype, int B, int n, int m, bool logd = false) {
   Choice best;
   const bool f32 = dtype == 0;
   const Tile* tab = f32 ? kTilesF32 : kTilesF64;
@@ -129,7 +136,8 @@ Choice choose(int dtype, int B, int n, int m) {
     double cost = 1100.0 + 2.0 * t.ER * t.EC * t.W * share;
     if (C > 1) cost += 3000.0 + 3.0 * t.rows() * C / t.W;
     if (R > 1) cost += 3000.0 + 3.0 * t.cols() * R / t.W;
-    if (best.tile < 0 || cost < best_cost) {
+    const bool fewer = R * C == 1 && (total > kCus || (logd && !f32));
+    if (best.tile < 0 || cost < best_cost || (fewer && cost == best_cost)) {
       best.tile = q;
       best.R = R;
       best.C = C;
@@ -174,7 +182,7 @@ size_t resident_workspace(int dtype, int B, int n, int m) {
 // were), other: a HIP error.
 int resident_solve(int dtype, ResidentArgs a, double* u_keep, double* v_keep, Ctrl* host_ctrl,
                    hipStream_t s, Ctrl* out) {
-  const Choice c = choose(a.stab ? 1 : dtype, a.B, a.n, a.m);
+  const Choice c = choose(a.stab ? 1 : dtype, a.B, a.n, a.m, a.logd && !a.stab);
   if (c.tile < 0) return 1;
   const bool f32 = dtype == 0 && !a.stab;  // (stabilised: fp64 elements)
   const Tile t = f32 ? kTilesF32[c.tile] : kTilesF64[c.tile];

@@ -56,8 +56,8 @@
 // domain, against 61 and 64 on the row sweep (36 and 38 where rows are
 // 16-byte aligned).)
 #define POTAMD_TILES_F32(X) \
-  X(4, 2, 4) X(4, 4, 4) X(8, 4, 8) X(8, 8, 8) X(8, 4, 16) X(8, 8, 16) X(8, 10, 20)
-#define POTAMD_TILES_F64(X) X(4, 2, 4) X(4, 4, 4) X(8, 2, 8) X(8, 4, 8) X(8, 8, 8) X(8, 4, 16)
+  X(4, 2, 4) X(4, 4, 4) X(8, 4, 8) X(4, 8, 8) X(8, 8, 8) X(8, 4, 16) X(8, 8, 16) X(8, 10, 20)
+#define POTAMD_TILES_F64(X) X(4, 2, 4) X(4, 4, 4) X(8, 2, 8) X(8, 4, 8) X(4, 8, 8) X(8, 8, 8) X(8, 4, 16)
 
 namespace potamd {
 namespace {

@@ -224,3 +224,10 @@ def test_many_values_to_exchange(n, m, dtype):
         if domain == _lib.SCALING:
             u, v = np.log(u), np.log(v)
         _check_plan(M[0], reg, u, v, P, dtype)
+
+
+@pytest.mark.parametrize("dtype", [F64, F32])
+@pytest.mark.parametrize("B,n,m", [(300, 128, 127), (257, 65, 66)])
+def test_more_problems_than_cus(B, n, m, dtype):
+    """Problems of 65 to 128 a side, two and more of them on a CU."""
+    test_batch_with_one_stop(B, n, m, dtype)
