@@ -271,6 +271,9 @@ def solve_gromov_batch(C1, C2, reg=1e-2, a=None, b=None, loss="sqeuclidean", sym
         T = ad[:, :, None] * bd[:, None, :] / scale[:, None, None]
     else:
         T = T_init.detach()
+    # (elementwise results keep their operands' strides: a start or a cost given
+    # as a transposed view would make the kernel of the projection one too)
+    T, Md = T.contiguous(), Md.contiguous()
     log_T = torch.log(T + EPS_LOG)
     proj, step = None, -1
     h1, h2 = _as_channels(Ld["hC1"]), _as_channels(Ld["hC2"])
@@ -284,7 +287,6 @@ def solve_gromov_batch(C1, C2, reg=1e-2, a=None, b=None, loss="sqeuclidean", sym
         many = isinstance(reg, torch.Tensor) and reg.numel() > 1  # a reg per problem
         gain = w if many else w / float(reg) if reg else float("inf")
         for step in range(max_iter):
-            T = T.contiguous()
             K = log_T - const
             S = torch.zeros_like(K) if many else K
             for d in range(h1.shape[-1]):
