@@ -261,6 +261,7 @@ def solve_gromov_batch(C1, C2, reg=1e-2, a=None, b=None, loss="sqeuclidean", sym
     if not isinstance(loss, str):
         raise ValueError(f"Unknown loss function: {loss}")
     L = tensor_batch(a, b, C1, C2, symmetric=symmetric, loss=loss, logits=logits)
+    fused = M is not None
     M, alpha = _check_fused(M, alpha, B, n, m, C1)
 
     # the outer loop sees detached data only
@@ -279,23 +280,27 @@ def solve_gromov_batch(C1, C2, reg=1e-2, a=None, b=None, loss="sqeuclidean", sym
     h1, h2 = _as_channels(Ld["hC1"]), _as_channels(Ld["hC2"])
     a64, b64 = ad.to(torch.float64).contiguous(), bd.to(torch.float64).contiguous()
     with torch.no_grad():
-        # log T - lin / reg, where lin = (1 - alpha) M + 2 alpha (constC - w S):
-        # the part that stays, then S added by the products themselves (the
-        # separable part of a product with zero marginals is not formed)
-        const = ((1 - alpha) * Md + (2 * alpha) * Ld["constC"]) / reg
-        w = 2.0 * float(alpha) * (1.0 if symmetric else 0.5)
-        many = isinstance(reg, torch.Tensor) and reg.numel() > 1  # a reg per problem
-        gain = w if many else w / float(reg) if reg else float("inf")
+        # log T - lin / reg, where lin = (1 - alpha) M + 2 alpha (constC - w S).
+        # The products are taken from constC itself: the two may cancel, so
+        # neither is scaled before (scaled by 2 alpha / reg first, the roundings
+        # of both stay: structures of 1000 + small integers, 1e-9 of the plan
+        # against 1e-14).
+        lin0 = (1 - alpha) * Md
+        w = -1.0 if symmetric else -0.5
+        two_alpha = 2.0 * (alpha.item() if isinstance(alpha, torch.Tensor) else float(alpha))
+        number = isinstance(reg, (int, float)) and reg != 0
         for step in range(max_iter):
-            K = log_T - const
-            S = torch.zeros_like(K) if many else K
+            lin = Ld["constC"].clone()
             for d in range(h1.shape[-1]):
                 h1d, h2d = h1[..., d], h2[..., d]
-                _solve.gemm(_solve.bmm(h1d, T), h2d, S, alpha=gain, beta=1.0, transB=True)
+                _solve.gemm(_solve.bmm(h1d, T), h2d, lin, alpha=w, beta=1.0, transB=True)
                 if not symmetric:
-                    _solve.gemm(_solve.bmm(h1d, T, transA=True), h2d, S, alpha=gain, beta=1.0)
-            if many:
-                K += S / reg
+                    _solve.gemm(_solve.bmm(h1d, T, transA=True), h2d, lin, alpha=w, beta=1.0)
+            if fused:
+                lin = torch.add(lin0, lin, alpha=two_alpha)
+                K = torch.sub(log_T, lin, alpha=1.0 / reg) if number else log_T - lin / reg
+            else:  # (alpha = 1)
+                K = torch.sub(log_T, lin, alpha=2.0 / reg) if number else log_T - 2.0 * lin / reg
             u0, v0 = _solve.start(B, n, m, 0.0, K.device)
             res = _solve.dense_solve(K, a64, b64, u0, v0, None, domain=_lib.LOG,
                                      order=_lib.ROW_FIRST, kernel_given=True,

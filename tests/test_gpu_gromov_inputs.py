@@ -51,3 +51,28 @@ def test_reg_per_problem():
         s = slice(p, p + 1)
         one = pb.solve_gromov_batch(C1[s], C2[s], reg=float(regs[p]), T_init=T[s], M=M[s], **kw)
         torch.testing.assert_close(got.plan[s], one.plan, rtol=1e-11, atol=1e-15)
+
+
+def test_products_that_cancel():
+    """Structures far from zero, whose products and constant part agree in all
+    but their last digits.  Both are sums of integers here, exact in float64, so
+    one step is a projection of exp(log T - lin / reg) with exponents up to 100:
+    some tens of roundings of 2^7 2^-53 in K, u and v, 1e-12 relative in the plan."""
+    rng = np.random.default_rng(7)
+    n = m = 8
+    C1 = 1000.0 + rng.integers(0, 5, (2, n, n))
+    C2 = 1000.0 + rng.integers(0, 5, (2, m, m))
+    C1, C2 = C1 + C1.transpose(0, 2, 1), C2 + C2.transpose(0, 2, 1)
+    reg = 0.3
+    T = np.full((2, n, m), 1.0 / (n * m))
+    # sum_jl (C1_ij - C2_kl)^2 T_jl, formed without cancellation
+    lin = 2.0 * np.einsum("bijkl->bik", (C1[:, :, :, None, None] - C2[:, None, None]) ** 2
+                          ) / (n * m)
+    K = np.log(T + 1e-15) - lin / reg
+    v = np.zeros((2, m))
+    for _ in range(30):
+        u = np.log(1.0 / n) - np.logaddexp.reduce(K + v[:, None, :], axis=2)
+        v = np.log(1.0 / m) - np.logaddexp.reduce(K + u[:, :, None], axis=1)
+    want = np.exp(K + u[:, :, None] + v[:, None, :])
+    got = pb.solve_gromov_batch(C1, C2, reg=reg, max_iter=1, max_iter_inner=30, tol_inner=0.0)
+    np.testing.assert_allclose(got.plan, want, rtol=1e-12, atol=1e-18)
