@@ -9,6 +9,7 @@
 //   sums[1] = sum P * log(P + 1e-16)     (-entropy_batch, _utils.py:4-22)
 //   sums[2] = sum P * log(P / (a b) + 1e-16)  (KL value, _linear.py:342-345)
 //   sums[3] = sum P
+// A plan has the same bits whether sums are asked for or not.
 // Bound: the plan alone reads the cost and writes P (16384^2 float32: 2.1 GB);
 // the sums are bound by the fp64 exponential and logarithms, so a logarithm is
 // taken only where its sum is asked for.
@@ -21,23 +22,6 @@ namespace potamd {
 
 constexpr int kPlanThreads = 256;
 constexpr int kPlanSums = 4;
-
-// 2^t to 2^-33 relative (the polynomial interpolates 2^r on [-1/2, 1/2] at the
-// Chebyshev nodes of degree 8): an fp32 result is rounded as from the exact
-// value, for half the instructions of exp().
-__device__ __forceinline__ double exp2_for_f32(double t) {
-  t = t < -1100.0 ? -1100.0 : (t > 1100.0 ? 1100.0 : t);  // infinities; a NaN stays
-  const double k = rint(t), r = t - k;
-  double y = 1.5303700711365693e-05;
-  y = fma(y, r, 0.00015469729214118296);
-  y = fma(y, r, 0.0013333478473685416);
-  y = fma(y, r, 0.009618025613318034);
-  y = fma(y, r, 0.055504109063258665);
-  y = fma(y, r, 0.24022651213498092);
-  y = fma(y, r, 0.6931471805568324);
-  y = fma(y, r, 0.9999999999595618);
-  return ldexp(y, (int)k);
-}
 
 // (aligned as its elements: rows of any width and stride move 16 bytes at a
 // time; an element at a time, a 5000 x 4999 float32 plan took 82 us, 50 now)
@@ -66,7 +50,6 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs A) {
   const double inv_reg = A.kernel_given ? 0.0 : 1.0 / A.reg;
   const bool logd = A.domain == kLog, given = A.kernel_given;
   const bool ent = SUMS && A.which & 2, kl = SUMS && A.which & 4;
-  const double s2 = given ? kLog2e : -kLog2e * inv_reg;
   double s_cost = 0, s_ent = 0, s_kl = 0, s_mass = 0;
   const int r0 = (blockIdx.x / A.csplit) * A.rpb, r1 = min(n, r0 + A.rpb);
   for (int jt = ((blockIdx.x % A.csplit) * TX + tx) * VEC; jt < m; jt += A.csplit * TX * VEC) {
@@ -99,14 +82,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs A) {
         for (int c = 0; c < VEC; ++c) {
           const double mij = (double)x[q].x[c];
           double pij, xij = 0.0;
-          if (!SUMS && sizeof(TM) == 4) {
-            if (logd) {
-              pij = exp2_for_f32(fma(mij, s2, (ui[q] + vj[c]) * kLog2e));
-              if (L) xij = (given ? mij : -mij * inv_reg) + ui[q] + vj[c];
-            } else {
-              pij = ui[q] * (given ? mij : exp2_for_f32(mij * s2)) * vj[c];
-            }
-          } else if (logd) {
+          if (logd) {
             xij = (given ? mij : -mij * inv_reg) + ui[q] + vj[c];
             pij = exp(xij);
           } else {
