@@ -527,7 +527,7 @@ __global__ __launch_bounds__(64 * W) void resident_kernel(ResidentArgs A) {
   }
   __syncthreads();
   if (LOG && !A.resume && !row_first) {
-    // v_1 = log b - LSE_i(M s2 + u_0), exactly.
+    // v_1 = log b - LSE_i(M s2 + u_0), in fp64 for either type.
     const int l = here(lane), c0 = l & 15, r0 = wv * 4 + (l >> 4);
     if (c0 < ER) ursh[r0 + TR * c0] = rown ? Ur_l : -__builtin_inf();
     __builtin_amdgcn_wave_barrier();
@@ -552,7 +552,7 @@ __global__ __launch_bounds__(64 * W) void resident_kernel(ResidentArgs A) {
     for (int k = 0; k < EC; ++k) acc[k] = 0.0;
 #pragma unroll 1
     for (int e = 0; e < ER; ++e)
-      exponents(e, [&](int k, double x) { acc[k] += (double)exp2_of(x - cmx[c0 + 16 * k], R()); });
+      exponents(e, [&](int k, double x) { acc[k] += exp2(x - cmx[c0 + 16 * k]); });
     double sm = cols_reduce(acc, Sum());
     if (GR > 1) sm = cols_of(sm, Sum());
     if (cown) {
