@@ -139,7 +139,11 @@ int plan_blocks(int n) { return (n + 7) / 8 + 8; }
 
 hipError_t launch_plan(int dtype, PlanArgs a, int B, double* sums, hipStream_t s) {
   const int wide = dtype == 0 ? 4 : 2;
-  const bool vec = a.m >= wide;
+  // A plan written over its cost takes an element at a time where rows do not
+  // end with a vector: the last one would read columns that its neighbour's
+  // thread may have written.
+  const bool over = a.P == a.M || a.logP == a.M;
+  const bool vec = a.m >= wide && !(over && a.m % wide != 0);
   const int v = vec ? wide : 1;
   a.tx = 3;
   while (a.tx < 8 && (v << a.tx) < a.m) ++a.tx;
