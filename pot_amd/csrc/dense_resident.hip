@@ -5,7 +5,9 @@
 #include <algorithm>
 #include <atomic>
 #include <chrono>
+#include <condition_variable>
 #include <mutex>
+#include <thread>
 
 #include "host.h"
 #include "internal.h"
@@ -163,11 +165,63 @@ Words words_of(int B, int n, int m, const Choice& c) {
   return w;
 }
 
-// Solves whose workgroups wait for each other run one at a time on a device.
-std::timed_mutex& waiting_solves(int dev) {
-  static std::timed_mutex locks[64];
-  return locks[dev & 63];
-}
+// Solves whose workgroups wait for each other, of all threads of the process on
+// one device: together they have at most a workgroup a CU, so that each finds a
+// CU that none of the others holds and all are resident (workgroups go to the
+// eight XCDs in turn, so a solve counts as a multiple of eight).  Other kernels
+// end by themselves.
+class WaitingSolves {
+  using Clock = std::chrono::steady_clock;
+
+ public:
+  // Notes a solve of this thread; whether another thread had one in the last second.
+  bool arrive() {
+    std::lock_guard<std::mutex> lock(mutex_);
+    const auto me = std::this_thread::get_id();
+    if (me != last_) others_at_ = last_at_;
+    last_ = me;
+    last_at_ = Clock::now();
+    return last_at_ - others_at_ < std::chrono::seconds(1);
+  }
+  // False where the CUs are not free for a second: the holders' streams share a
+  // hardware queue with longer work.
+  bool enter(int cus, int of) {
+    std::unique_lock<std::mutex> lock(mutex_);
+    if (!freed_.wait_for(lock, std::chrono::seconds(1),
+                         [&] { return used_ == 0 || used_ + cus <= of; }))
+      return false;
+    used_ += cus;
+    return true;
+  }
+  void leave(int cus) {
+    {
+      std::lock_guard<std::mutex> lock(mutex_);
+      used_ -= cus;
+    }
+    freed_.notify_all();
+  }
+  static WaitingSolves& on(int dev) {
+    static WaitingSolves* all = new WaitingSolves[64];  // (outlives every thread)
+    return all[dev & 63];
+  }
+
+ private:
+  std::mutex mutex_;
+  std::condition_variable freed_;
+  int used_ = 0;
+  std::thread::id last_;  // the last solve's thread, and when; the last of another one
+  Clock::time_point last_at_ = Clock::time_point() - std::chrono::hours(1);
+  Clock::time_point others_at_ = last_at_;
+};
+
+// The CUs of one solve, until it has ended.
+struct CuShare {
+  WaitingSolves* of = nullptr;
+  int cus = 0;
+  ~CuShare() {
+    if (of) of->leave(cus);
+  }
+};
 
 }  // namespace
 
@@ -224,12 +278,20 @@ int resident_solve(int dtype, ResidentArgs a, double* u_keep, double* v_keep, Ct
   Ctrl local;
   Ctrl* hc = host_ctrl ? host_ctrl : &local;
 
-  std::unique_lock<std::timed_mutex> only;
+  CuShare share;
   if (waits) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return 1;
-    only = std::unique_lock<std::timed_mutex>(waiting_solves(dev), std::defer_lock);
-    if (!only.try_lock_for(std::chrono::seconds(1))) return 1;
+    WaitingSolves& solves = WaitingSolves::on(dev);
+    // Where several threads solve, the CUs are held for the solve alone, not for
+    // work queued before it (another thread's solve would wait for that).  A
+    // program of one thread queues the solve behind that work: 2048^2 float64
+    // 451 us a call, 494 with the wait.
+    if (solves.arrive() && hipStreamSynchronize(s) != hipSuccess) return -1;
+    const int cus = std::min(device_cus(), (grid + 7) / 8 * 8);
+    if (!solves.enter(cus, device_cus())) return 1;
+    share.of = &solves;
+    share.cus = cus;
   }
   if (!lone) {
     const int64_t words = waits ? w.total : 0;

@@ -32,10 +32,10 @@
 // all hold the same sums and take the same decisions.
 //
 // Workgroups that wait for each other have to be resident together: the host
-// launches at most what fits the GPU, one such solve at a time, and every
-// wait is bounded (then the solve is abandoned and repeated by dense.hip, as
-// it is where a scaling is not finite or a column mass falls below the
-// trusted range, whose outcome dense.hip reports).
+// launches at most what fits the GPU, several solves at a time only where they
+// fit together, and every wait is bounded (then the solve is abandoned and
+// repeated by dense.hip, as it is where a scaling is not finite or a column
+// mass falls below the trusted range, whose outcome dense.hip reports).
 //
 // The stabilised solver (sinkhorn_stabilized) is the scaling domain on
 // K = exp((alpha + beta - M) / reg) in fp64, kept in the cost's type, with
