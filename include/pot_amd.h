@@ -55,6 +55,13 @@ size_t potamd_dense_workspace_size(int dtype, int batch, int n, int m, int rows_
  * whose tile the caller may then choose. */
 int potamd_dense_resident(int dtype, int batch, int n, int m);
 
+/* Longest wait of a workgroup for another of its solve, in microseconds, in the
+ * solves that the calling thread starts from now on: 0 is the default (20000),
+ * a negative value makes the third wait give up at once.  A solve that gave up
+ * is repeated on the row sweep, and for half a second the device's solves go
+ * ways that do not wait; this call ends that time. */
+int potamd_resident_wait_limit(int us);
+
 /* Dense-cost Sinkhorn on `batch` problems of shape n x m sharing one reg.
  *
  * Replaces the iteration loops of

@@ -24,6 +24,7 @@ SIGNATURES = {
     "potamd_status_string": (ctypes.c_char_p, [c_int]),
     "potamd_dense_workspace_size": (c_size, [c_int, c_int, c_int, c_int, c_int]),
     "potamd_dense_resident": (c_int, [c_int, c_int, c_int, c_int]),
+    "potamd_resident_wait_limit": (c_int, [c_int]),
     "potamd_sinkhorn_dense": (c_int, [
         c_int, c_int, c_int, c_int,          # dtype, domain, order, kernel_given
         c_vp, c_i64, c_i64, c_int, c_int, c_int,  # M, ldm, bstride, batch, n, m

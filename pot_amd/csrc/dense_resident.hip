@@ -9,6 +9,7 @@
 #include <mutex>
 #include <thread>
 
+#include "../../include/pot_amd.h"
 #include "host.h"
 #include "internal.h"
 #include "resident.h"
@@ -193,6 +194,17 @@ class WaitingSolves {
     used_ += cus;
     return true;
   }
+  // Whether solves that wait are left out now: after a wait that ran out, for half
+  // a second (what keeps workgroups off the GPU may do so at each call, and each
+  // would lose those 20 ms).
+  bool paused() {
+    std::lock_guard<std::mutex> lock(mutex_);
+    return Clock::now() < paused_until_;
+  }
+  void pause(std::chrono::milliseconds time) {
+    std::lock_guard<std::mutex> lock(mutex_);
+    paused_until_ = Clock::now() + time;
+  }
   void leave(int cus) {
     {
       std::lock_guard<std::mutex> lock(mutex_);
@@ -212,6 +224,7 @@ class WaitingSolves {
   std::thread::id last_;  // the last solve's thread, and when; the last of another one
   Clock::time_point last_at_ = Clock::time_point() - std::chrono::hours(1);
   Clock::time_point others_at_ = last_at_;
+  Clock::time_point paused_until_ = last_at_;
 };
 
 // The CUs of one solve, until it has ended.
@@ -222,6 +235,8 @@ struct CuShare {
     if (of) of->leave(cus);
   }
 };
+
+thread_local long long wait_ticks = kWaitTicks;
 
 }  // namespace
 
@@ -257,15 +272,19 @@ int resident_solve(int dtype, ResidentArgs a, double* u_keep, double* v_keep, Ct
   // problems of a batch with one stop, unless there are more than fit.
   const bool blocked = c.R * c.C > 1, joint = a.B > 1 && !a.each;
   bool segment = false, waits = blocked || joint;
+  a.wait_ticks = wait_ticks;
   size_t lds = lds_bytes(t, c.R, c.C, waits ? (a.each ? 1 : a.B) * parts : 0);
   auto launch = [&](const ResidentArgs& x, int* per_cu) -> hipError_t {
     if (x.stab) return resident_launch_stab(dtype == 0, t, x, grid, lds, s, per_cu);
     return f32 ? resident_launch_f32(t, x, grid, lds, s, per_cu)
                : resident_launch_f64(t, x, grid, lds, s, per_cu);
   };
+  int dev = 0;
   if (waits) {
+    if (hipGetDevice(&dev) != hipSuccess) return 1;
     int per_cu = 0;
-    const bool fits = lds <= 160 * 1024 && launch(a, &per_cu) == hipSuccess &&
+    const bool fits = !WaitingSolves::on(dev).paused() && lds <= 160 * 1024 &&
+                      launch(a, &per_cu) == hipSuccess &&
                       (int64_t)grid <= (int64_t)per_cu * device_cus();
     if (!fits) {
       if (blocked) return 1;
@@ -280,8 +299,6 @@ int resident_solve(int dtype, ResidentArgs a, double* u_keep, double* v_keep, Ct
 
   CuShare share;
   if (waits) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return 1;
     WaitingSolves& solves = WaitingSolves::on(dev);
     // Where several threads solve, the CUs are held for the solve alone, not for
     // work queued before it (another thread's solve would wait for that).  A
@@ -325,7 +342,7 @@ int resident_solve(int dtype, ResidentArgs a, double* u_keep, double* v_keep, Ct
          hipMemcpyAsync(hc, a.ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, s) != hipSuccess) ||
         hipStreamSynchronize(s) != hipSuccess)
       return -1;
-    if (a.host && !hc->done) hc->counter = 1;
+    if (a.host && !hc->done && !hc->counter) hc->counter = kGivenUp;
   } else {
     // One launch per check interval; the state travels in u and v themselves
     // (base 2), and at most two intervals are queued past an unread decision.
@@ -377,6 +394,8 @@ int resident_solve(int dtype, ResidentArgs a, double* u_keep, double* v_keep, Ct
   *out = *hc;
   if (a.each) out->status = out->niter >= a.max_iter - 1 ? kMaxIter : kConverged;
   if (!out->counter) return 0;
+  if (out->counter == kWaitedOut && waits)
+    WaitingSolves::on(dev).pause(std::chrono::milliseconds(500));
   // (the stabilised solve starts from alpha and beta, the others from u and v)
   double* const u_back = a.stab ? a.alpha_out : a.u_out;
   double* const v_back = a.stab ? a.beta_out : a.v_out;
@@ -387,3 +406,13 @@ int resident_solve(int dtype, ResidentArgs a, double* u_keep, double* v_keep, Ct
 }
 
 }  // namespace potamd
+
+using namespace potamd;
+
+extern "C" int potamd_resident_wait_limit(int us) {
+  wait_ticks = us == 0 ? kWaitTicks : us < 0 ? -1 : 100ll * us;
+  int dev = 0;
+  HIP_TRY(hipGetDevice(&dev));
+  WaitingSolves::on(dev).pause(std::chrono::milliseconds(0));
+  return 0;
+}

@@ -78,8 +78,9 @@ struct ResidentArgs {
   unsigned long long* words;  // exchange slots
   int row_slot, col_slot;
   int64_t err_slot, col_base, err_base;
-  Ctrl* ctrl;
-  Ctrl* host;  // pinned, device-visible: the outcome (or null: it is in ctrl)            // counter != 0: abandoned
+  Ctrl* ctrl;            // counter != 0: abandoned
+  Ctrl* host;            // pinned, device-visible: the outcome (or null: it is in ctrl)
+  long long wait_ticks;  // longest wait; < 0: the third wait gives up
   // stabilised: u_in / v_in hold alpha / beta
   int stab, period;
   double reg, inv_reg, tau, u_start, v_start;

@@ -62,7 +62,12 @@
 namespace potamd {
 namespace {
 
-constexpr long long kSpinTicks = 20000000;  // 0.2 s of the 100 MHz clock
+// Longest wait, in ticks of the 100 MHz clock: 20 ms.  The members of an exchange
+// are some microseconds apart (a member that forms K again tens), so a wait that
+// lasts is for a workgroup that another process or a long kernel keeps off the GPU.
+constexpr long long kWaitTicks = 2000000;
+// Ctrl::counter of a solve that was given up: by its numbers, or by a wait.
+constexpr unsigned kGivenUp = 1, kWaitedOut = 2;
 
 typedef unsigned long long word_t;
 
@@ -175,7 +180,7 @@ __global__ __launch_bounds__(64 * W) void resident_kernel(ResidentArgs A) {
   R* gsh = reinterpret_cast<R*>(ursh + RB);
   double* xs = ursh + RB + CB;     // exchanged values
   __shared__ double red[W];
-  __shared__ int dead;    // a wait gave up
+  __shared__ int dead;    // a wait ended: 1 another workgroup gave up, 2 too long
   // Of the column update: 1 references move, 2 abandon.  Stabilised: a scaling
   // over tau, of columns 4 and 16 in turn (a wave may be a column update ahead
   // of one that reads the last one's), of rows 8.
@@ -232,6 +237,10 @@ __global__ __launch_bounds__(64 * W) void resident_kernel(ResidentArgs A) {
   auto poll = [&](auto bytes, rsrc_t rsrc, int units, bool pause, unsigned tag, auto at, auto take) {
     constexpr int Q = ER == 10 ? 5 : 4;  // reads of a thread in flight
     using V = typename std::conditional<decltype(bytes)::value == 16, u32x4, u32x2>::type;
+    if (A.wait_ticks < 0 && tag >= 3) {  // (as potamd_resident_wait_limit asked)
+      dead = 2;
+      return;
+    }
     if (pause) __builtin_amdgcn_s_sleep(8);
     for (int w0 = tid; w0 < units; w0 += Q * T) {
       V v[Q];
@@ -257,9 +266,10 @@ __global__ __launch_bounds__(64 * W) void resident_kernel(ResidentArgs A) {
           if ((spin & 63) == 63) {
             const long long now = wall_clock64();
             if (since == 0) since = now;
-            if (__hip_atomic_load(&A.ctrl->counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ||
-                now - since > kSpinTicks) {
-              dead = 1;
+            const bool told = dead || __hip_atomic_load(&A.ctrl->counter, __ATOMIC_RELAXED,
+                                                        __HIP_MEMORY_SCOPE_AGENT);
+            if (told || now - since > A.wait_ticks) {
+              if (!dead) dead = told ? 1 : 2;
               break;
             }
           }
@@ -368,8 +378,11 @@ __global__ __launch_bounds__(64 * W) void resident_kernel(ResidentArgs A) {
   };
   auto abandon = [&]() {
     if (tid == 0) {
-      __hip_atomic_store(&A.ctrl->counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (A.host) A.host->counter = 1;
+      if (dead != 1) {  // (else the cause stands there)
+        const unsigned why = dead == 2 ? kWaitedOut : kGivenUp;
+        __hip_atomic_store(&A.ctrl->counter, why, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (A.host) A.host->counter = why;
+      }
       if (A.segment) A.ctrl->done = 1;
     }
   };
