@@ -98,7 +98,14 @@ constexpr int kSplitMax = 8;
 constexpr size_t kSplitCols = 256;                                    // byte offset
 constexpr size_t kSplitDbl = kSplitCols + 2ull * kSplitMax * kPMax * 4;  // byte offset
 constexpr size_t kSplitSlot = kSplitDbl + 256;
-constexpr int kSplitSpin = 1 << 22;  // polls (with a sleep each) before giving up
+// Polls (with a sleep each, half a microsecond and more) before giving up: for
+// parts that are all at work, some seconds.  A part that is still in the queue is
+// taken when a workgroup is done with its problem, so at the first exchange the
+// count starts again whenever the queue has moved, and allows kSplitTurn polls for
+// each iteration that a problem may take (at most 60 us; an unsplit problem of
+// 1024 points takes 44).
+constexpr int kSplitSpin = 1 << 22;
+constexpr int kSplitTurn = 256;
 static_assert(kSplitSlot == kPointsSplitSlot && kSplitCols == kPointsSplitCounters,
               "internal.h states the split slot layout");
 
@@ -336,10 +343,17 @@ __device__ __forceinline__ void solve_points(const PointsArgs& A, PointsLds<PW>&
       __atomic_signal_fence(__ATOMIC_SEQ_CST);
       __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       const int target = K * (sgen + 1);
-      int ok = 1;
+      const int turns = A.max_iter < (1 << 22) ? A.max_iter : 1 << 22;
+      const int most = sgen == 0 ? kSplitSpin + kSplitTurn * turns : kSplitSpin;
+      int ok = 1, head = 0;
       for (int spin = 0;
            __hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target; ++spin) {
-        if (spin >= kSplitSpin) {
+        if (sgen == 0) {
+          const int now = __hip_atomic_load(&A.queue[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          if (now != head) spin = 0;
+          head = now;
+        }
+        if (spin >= most) {
           ok = 0;
           break;
         }

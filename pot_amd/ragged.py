@@ -420,7 +420,9 @@ def auto_plan(ns, ms, cus=None):
     and up unsplit, 27 in two parts; 4096: 30 to 53, 36).
 
     The parts of a problem follow each other in the queue, so a part waits at
-    most for workgroups on earlier problems, whose parts are all taken."""
+    most for workgroups on earlier problems, whose parts are all taken.  Before
+    all parts have met, that wait ends (status 2) only where the queue has stood
+    still for longer than a problem's numItermax iterations can take."""
     ns = np.asarray(ns, dtype=np.int64)
     ms = np.asarray(ms, dtype=np.int64)
     nm = ns * ms
