@@ -1,4 +1,5 @@
-"""Split point-cloud problems whose parts wait for a workgroup."""
+"""Split point-cloud problems whose parts wait for a workgroup, and the calls
+that launch them without a host wait."""
 
 import numpy as np
 import pytest
@@ -29,3 +30,20 @@ def test_a_part_waits_as_long_as_earlier_problems_take():
     assert res.status[-1].item() == 0 and res.niter[-1].item() == 0
     u, v = res.split(P, B - 1)
     np.testing.assert_allclose((u[:, None] + v[None]).cpu().numpy(), -2 * np.log(128), rtol=1e-6)
+
+
+def _uneven(B):
+    rng = np.random.default_rng(B)
+    ns, ms = rng.integers(300, 512, B), rng.integers(300, 512, B)
+    xs = torch.tensor(rng.standard_normal((ns.sum(), 4)), dtype=torch.float32, device="cuda")
+    ys = torch.tensor(rng.standard_normal((ms.sum(), 4)), dtype=torch.float32, device="cuda")
+    return ns, ms, xs, ys, np.exp(rng.uniform(np.log(0.02), np.log(0.1), B))
+
+
+def test_a_split_graph_returns_before_its_replay_ends():
+    ns, ms, xs, ys, regs = _uneven(600)
+    G = ragged.RaggedGraph(ns, ms, 4, numItermax=4000, stopThr=0.0, cost="points")
+    assert G.parts is not None
+    G.solve(xs, ys, regs)
+    assert not torch.cuda.current_stream().query()
+    torch.cuda.synchronize()
