@@ -260,6 +260,7 @@ class RaggedPoints:
     regs_host: np.ndarray = None  # (B,) float64 host copy of regs (launch order)
     cmax: torch.Tensor = None  # (B,) float64 cost maxima once found (points_cmax)
     order: torch.Tensor = None  # (B,) int32 longest-first launch order, on the device
+    order_host: np.ndarray = None  # the same on the host (the queue of split problems)
 
     @property
     def batch(self):
@@ -334,7 +335,8 @@ def points_from_clouds(xs, ys, regs, a=None, b=None, normalize=True, device=None
                         Y=_pack_points(ys, device), aoff=t64[0:B], boff=t64[B:2 * B],
                         ns_d=t32[0:B], ms_d=t32[B:2 * B], a=_weights(a, ns, device),
                         b=_weights(b, ms, device), regs=t64[2 * B:3 * B].view(torch.float64),
-                        normalize=bool(normalize), regs_host=regs_h, order=t32[2 * B:3 * B])
+                        normalize=bool(normalize), regs_host=regs_h, order=t32[2 * B:3 * B],
+                        order_host=h32[2 * B:3 * B].copy())
 
 
 def _check_order(order, B):
@@ -472,6 +474,11 @@ def _split_items(order, parts):
     first = np.repeat(np.cumsum(reps) - reps, reps)
     part = np.arange(len(probs)) - first
     return (probs | (part << 24)).astype(np.int32)
+
+
+def _upload(x, dev):
+    """Host array to the device from pinned memory, without a host wait."""
+    return torch.from_numpy(x).pin_memory().to(dev, non_blocking=True)
 
 
 def _warn_unsolved(status):
@@ -613,13 +620,16 @@ def sinkhorn_log_ragged_points(P, u0=None, numItermax=1000, stopThr=1e-9, order=
     given = cmax is not None and P.normalize
     cmax = cmax.to(device=dev, dtype=torch.float64).contiguous() if given \
         else torch.empty(B, dtype=torch.float64, device=dev)
+    order_h = None
     if order is None and P.order is not None:
-        order = P.order
+        order, order_h = P.order, P.order_host
     elif order is None:
         regs_h = P.regs_host if P.regs_host is not None else P.regs.cpu().numpy()
-        order = torch.from_numpy(_points_order(P.ns, P.ms, regs_h)).to(dev)
+        order_h = _points_order(P.ns, P.ms, regs_h)
+        order = torch.from_numpy(order_h).to(dev)
     else:
-        order = torch.as_tensor(_check_order(order, B), device=dev)
+        order_h = _check_order(order, B)
+        order = torch.as_tensor(order_h, device=dev)
     waves = _tuned("points", P.ns, P.ms, P.d, waves)[0]
     # work-queue counters of the persistent launch (the kernel leaves them zero)
     queue = torch.zeros(2, dtype=torch.int32, device=dev)
@@ -632,10 +642,14 @@ def sinkhorn_log_ragged_points(P, u0=None, numItermax=1000, stopThr=1e-9, order=
             else _check_parts(split, P.ns)
     if parts is not None and (parts > 1).any():
         table, nsplit = _split_tables(parts)
-        items = torch.from_numpy(_split_items(order.cpu().numpy(), parts)).to(dev)
+        if order_h is None:
+            order_h = order.cpu().numpy()
+        # (one upload, without a host wait for the work queued before)
+        both = _upload(np.concatenate([_split_items(order_h, parts), table]), dev)
+        items, table = both[:-B], both[-B:]
         sws = _split_workspace(lib, nsplit, dev)
         _launch_points_split(lib, P, P.X, P.Y, P.regs, u, v, niter, status, e_last, e_first,
-                             cmax, items, torch.from_numpy(table).to(dev), nsplit, sws,
+                             cmax, items, table, nsplit, sws,
                              numItermax, check_every, stopThr, fallback_thr,
                              ctypes.c_void_p(_device.stream_ptr(dev)), queue, cmax_given=given)
     else:

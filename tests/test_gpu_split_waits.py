@@ -40,6 +40,23 @@ def _uneven(B):
     return ns, ms, xs, ys, np.exp(rng.uniform(np.log(0.02), np.log(0.1), B))
 
 
+def test_a_split_solve_returns_without_a_wait():
+    """unsolved="nan": work queued before the call is still running when it returns."""
+    ns, ms, xs, ys, regs = _uneven(600)
+    assert ragged.auto_plan(ns, ms).max() > 1
+    P = ragged.points_from_clouds(list(xs.split(ns.tolist())), list(ys.split(ms.tolist())), regs)
+    kw = dict(numItermax=20, stopThr=0.0, unsolved="nan")
+    want = ragged.sinkhorn_log_ragged_points(P, **kw)
+    torch.cuda.synchronize()
+    torch.cuda._sleep(50_000_000)
+    before = torch.cuda.Event()
+    before.record()
+    got = ragged.sinkhorn_log_ragged_points(P, **kw)
+    assert not before.query()
+    torch.cuda.synchronize()
+    assert torch.equal(got.u, want.u) and torch.equal(got.v, want.v)
+
+
 def test_a_split_graph_returns_before_its_replay_ends():
     ns, ms, xs, ys, regs = _uneven(600)
     G = ragged.RaggedGraph(ns, ms, 4, numItermax=4000, stopThr=0.0, cost="points")
