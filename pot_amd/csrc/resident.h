@@ -163,8 +163,11 @@ __device__ __forceinline__ float exp2_of(double x, float) {
 // Scaling domain, log domain, stabilised (see above).
 enum ResidentMode { kResScaling, kResLog, kResStab };
 
+// (Two waves a SIMD: eight waves need that, and of the tiles of four, two
+// workgroups of the largest then share a CU.  Without it the float64 log solve
+// of 128 x 128 took 258 registers: 257 problems of 100^2 293 us, 236 with two.)
 template <typename TM, typename R, int W, int ER, int EC, int MODE, bool BLK>
-__global__ __launch_bounds__(64 * W) void resident_kernel(ResidentArgs A) {
+__global__ __launch_bounds__(64 * W, 2) void resident_kernel(ResidentArgs A) {
   constexpr bool LOG = MODE == kResLog, STAB = MODE == kResStab;
   constexpr int T = 64 * W, TR = 4 * W, RB = TR * ER, CB = 16 * EC;
   static_assert(ER <= 16 && EC % 4 == 0 && CB <= T, "tile");
