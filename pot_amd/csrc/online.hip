@@ -223,16 +223,34 @@ struct OnlineMergeArgs {
 struct Lse {
   double mx, acc;
 };
+// s0 and s1 are a wave's.  Sixteen at a time, each read once: the partials are
+// read past the caches, a microsecond a turn.
 template <typename Get>
 __device__ __forceinline__ Lse lse_of(int s0, int s1, Get get) {
+  constexpr int Q = 16;
+  s0 = __builtin_amdgcn_readfirstlane(s0);
+  s1 = __builtin_amdgcn_readfirstlane(s1);
   Lse x = {-__builtin_inf(), 0.0};
-#pragma unroll 8
-  for (int s = s0; s < s1; ++s) x.mx = fmax(x.mx, get(s));
-  if (x.mx > -__builtin_inf()) {
-#pragma unroll 8
-    for (int s = s0; s < s1; ++s) x.acc += exp2(get(s) - x.mx);
-  } else {
-    for (int s = s0; s < s1; ++s) x.acc = get(s) != get(s) ? __builtin_nan("") : x.acc;
+  for (int s = s0; s < s1; s += Q) {
+    const int k = s1 - s;
+    double v[Q], top = x.mx;
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+      if (q < k) v[q] = get(s + q);
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+      if (q < k) top = fmax(top, v[q]);
+    if (top > -__builtin_inf()) {
+      if (x.mx > -__builtin_inf()) x.acc *= exp2(x.mx - top);
+      x.mx = top;
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+        if (q < k) x.acc += exp2(v[q] - top);
+    } else {
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+        if (q < k && v[q] != v[q]) x.acc = v[q];
+    }
   }
   return x;
 }
