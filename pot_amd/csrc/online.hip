@@ -322,10 +322,15 @@ __device__ __forceinline__ void mma_chunk(f32x16& acc, u32x4 a, u32x4 b) {
 // 1.8e-7: 9 roundings of full size for 32).  16384^2 points, d = 64: 201 us a
 // pass, 313 before; matrix cores 46% busy, VALU 37%.  d <= 16 takes one K step
 // of 16 instead of two: 5000 x 4000 points in 3-D, 14.9 us a pass, 22 before.
-template <int P, int D, int MODE>
+// FEW: no more than two workgroups a CU in the launch, so that no more than two
+// waves a SIMD are of use: the scheduler then keeps more reads in flight.  (fp8,
+// d = 128, us a pass with / without: 1000^2 11.4 / 12.3, 3000 x 2500 13.2 / 13.9;
+// with more workgroups three waves are worth more, 9000^2 44.5 / 39.2.  The other
+// operands' passes have as many waves either way.)
+template <int P, int D, int MODE, bool FEW = false>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(
     ((P == POTAMD_ONLINE_BF16X3 && D == 64) || (P == POTAMD_ONLINE_F32 && D <= 64)) && MODE == kModeLse
-        ? 3 : 1)))
+        ? 3 : 1, FEW ? 2 : 8)))
 void online_pass_kernel(PassArgs A) {
   if (A.ctrl && A.ctrl->done) return;
   constexpr int es = Op<P>::es;
@@ -1214,7 +1219,14 @@ hipError_t launch_pass_d(int D, const PassArgs& a, int S, hipStream_t s) {
     case 32: hipLaunchKernelGGL((online_pass_kernel<P, 32, MODE>), grid, dim3(T), 0, s, a); break;
     case 64: hipLaunchKernelGGL((online_pass_kernel<P, 64, MODE>), grid, dim3(T), 0, s, a); break;
     case 96: hipLaunchKernelGGL((online_pass_kernel<P, 96, MODE>), grid, dim3(T), 0, s, a); break;
-    default: hipLaunchKernelGGL((online_pass_kernel<P, 128, MODE>), grid, dim3(T), 0, s, a); break;
+    default:
+      if constexpr (P == POTAMD_ONLINE_FP8)
+        if ((int)grid.x * S <= 2 * device_cus()) {
+          hipLaunchKernelGGL((online_pass_kernel<P, 128, MODE, true>), grid, dim3(T), 0, s, a);
+          break;
+        }
+      hipLaunchKernelGGL((online_pass_kernel<P, 128, MODE>), grid, dim3(T), 0, s, a);
+      break;
   }
   return hipGetLastError();
 }
