@@ -394,7 +394,7 @@ def split_plan(ns, ms, cus=None, regs=None):
     return parts
 
 
-# Size tiers of the automatic split: the least elements for 2, 4 and 8 parts.
+# Size tiers of ``auto_plan``: the least elements for 2, 4 and 8 parts.
 _NEVER = 1 << 62
 _TIERS = ((_NEVER, _NEVER, _NEVER), (1 << 17, _NEVER, _NEVER), (1 << 16, _NEVER, _NEVER),
           (1 << 17, 3 << 17, _NEVER), (1 << 16, 1 << 17, _NEVER), (1 << 17, 3 << 17, 3 << 18),
@@ -405,21 +405,25 @@ _FIXED_US = {1: 6.9, 2: 8.2, 4: 8.4, 8: 10.0}
 
 
 def auto_plan(ns, ms, cus=None):
-    """Workgroups per problem of the automatic split: the size tiers that make
-    the time of the GPU's work or of the longest problem, whichever is larger,
-    and half the other least.
+    """Workgroups per problem (for ``split=``) of a batch some of whose problems
+    need many times the iterations of the others: the size tiers that make the
+    time of the GPU's work or of the longest problem, whichever is larger, and
+    half the other least.
 
     The work is the parts' microseconds an iteration over the CUs.  The longest
     problem is the slowest one's iteration times 0.35 sqrt(B): over batches of
-    Gaussian clouds the most iterations were 4 (40 problems) to 24 (3000) times
-    their mean, and which problem needs them is not known, so problems of one
-    size are split alike.  (A budget of one part a CU left the chip waiting for
-    unsplit problems.)  Milliseconds unsplit / with that budget / now: 512
-    problems of 64 to 1024 points 10.4 / 5.5 / 4.9, 300 of 200 to 900 16.8 / 17.1 /
-    9.9, 100 of 64 to 1024 5.1 / 2.4 / 2.0; 256 of 1024 points 18.3 / 18.8 / 7.5,
-    512 14.4 / 14.8 / 6.1, 2000 33.2 / - / 19.5.  Past 8 problems a CU the work of
-    two parts is as long as most batches' longest problem (3000 of 1024 points: 23
-    and up unsplit, 27 in two parts; 4096: 30 to 53, 36).
+    mixtures at regs of 5e-3 to 5e-2 the most iterations were 4 (40 problems) to
+    24 (3000) times their mean, and which problem needs them is not known, so
+    problems of one size are split alike.
+
+    Not the automatic split, as parts cost work, and a batch whose problems take
+    about as many iterations each is bound by that.  Milliseconds at those regs,
+    unsplit / ``split_plan`` / so: 256 problems of 1024 points 86 / 87 / 33, 512 25 / 25 / 11,
+    1000 of 64 to 1024 38 / 38 / 19, 200 8.3 / 4.3 / 3.7, 512 16 / 7.3 / 9.2; 40 iterations
+    each, 1000 of 300 to 700 3.4 / 3.4 / 7.3, 513 of 100 to 500 1.2 / 1.2 / 1.7, 300 of 200
+    to 600 1.5 / 1.7 / 2.0.  Past 8 problems a CU the work of two parts is as long as
+    most batches' longest problem (3000 of 1024 points: 23 and up unsplit, 27 in two
+    parts; 4096: 30 to 53, 36).
 
     The parts of a problem follow each other in the queue, so a part waits at
     most for workgroups on earlier problems, whose parts are all taken.  Before
@@ -594,8 +598,8 @@ def sinkhorn_log_ragged_points(P, u0=None, numItermax=1000, stopThr=1e-9, order=
     sweep and never stored.  ``cmax``: the maxima from ``points_cmax`` (the
     solve then skips its own search).  ``waves``: wavefronts per problem (8
     or 16; 0 = the autotuned value of this batch class, else the library
-    default).  ``split``: "auto" (``auto_plan``: large problems of
-    batches whose longest would outlast the rest), None (one workgroup per problem) or workgroups
+    default).  ``split``: "auto" (``split_plan``: only batches too small to
+    fill the GPU are split), None (one workgroup per problem) or workgroups
     per problem (1..8): a split problem's rows are shared by several
     workgroups (8 waves each).  ``unsolved``: "dense" (default) solves the
     problems the kernel cannot take (status 2: scaled coordinates outside its
@@ -638,7 +642,7 @@ def sinkhorn_log_ragged_points(P, u0=None, numItermax=1000, stopThr=1e-9, order=
         # (sizes only, as RaggedGraph plans before it sees the regs, so the
         # eager solve and a graph replay of one batch split alike and agree
         # bit for bit)
-        parts = auto_plan(P.ns, P.ms) if (isinstance(split, str) and split == "auto") \
+        parts = split_plan(P.ns, P.ms) if (isinstance(split, str) and split == "auto") \
             else _check_parts(split, P.ns)
     if parts is not None and (parts > 1).any():
         table, nsplit = _split_tables(parts)
@@ -719,7 +723,7 @@ class RaggedGraph:
         # the queue items re-ordered on each solve, the exchange slots zero.
         self.parts = None
         if split is not None and cost == "points":
-            parts = auto_plan(self.ns, self.ms) if (isinstance(split, str) and split == "auto") \
+            parts = split_plan(self.ns, self.ms) if (isinstance(split, str) and split == "auto") \
                 else _check_parts(split, self.ns)
             if (parts > 1).any():
                 self.parts = parts

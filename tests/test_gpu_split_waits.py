@@ -43,9 +43,10 @@ def _uneven(B):
 def test_a_split_solve_returns_without_a_wait():
     """unsolved="nan": work queued before the call is still running when it returns."""
     ns, ms, xs, ys, regs = _uneven(600)
-    assert ragged.auto_plan(ns, ms).max() > 1
+    parts = ragged.auto_plan(ns, ms)
+    assert parts.max() > 1
     P = ragged.points_from_clouds(list(xs.split(ns.tolist())), list(ys.split(ms.tolist())), regs)
-    kw = dict(numItermax=20, stopThr=0.0, unsolved="nan")
+    kw = dict(numItermax=20, stopThr=0.0, unsolved="nan", split=parts)
     want = ragged.sinkhorn_log_ragged_points(P, **kw)
     torch.cuda.synchronize()
     torch.cuda._sleep(50_000_000)
@@ -59,8 +60,19 @@ def test_a_split_solve_returns_without_a_wait():
 
 def test_a_split_graph_returns_before_its_replay_ends():
     ns, ms, xs, ys, regs = _uneven(600)
-    G = ragged.RaggedGraph(ns, ms, 4, numItermax=4000, stopThr=0.0, cost="points")
+    G = ragged.RaggedGraph(ns, ms, 4, numItermax=4000, stopThr=0.0, cost="points",
+                           split=ragged.auto_plan(ns, ms))
     assert G.parts is not None
     G.solve(xs, ys, regs)
     assert not torch.cuda.current_stream().query()
     torch.cuda.synchronize()
+
+
+def test_the_automatic_split_leaves_full_batches_whole():
+    """More than two problems a CU: parts would only add work where the problems
+    take about as many iterations each."""
+    ns, ms, xs, ys, regs = _uneven(600)
+    G = ragged.RaggedGraph(ns, ms, 4, numItermax=20, stopThr=0.0, cost="points")
+    assert G.parts is None
+    G = ragged.RaggedGraph(ns[:90], ms[:90], 4, numItermax=20, stopThr=0.0, cost="points")
+    np.testing.assert_array_equal(G.parts, ragged.split_plan(ns[:90], ms[:90]))
