@@ -727,10 +727,6 @@ class RaggedGraph:
                 else _check_parts(split, self.ns)
             if (parts > 1).any():
                 self.parts = parts
-                # Small batches are looked over for problems left unsolved, which
-                # waits for the replay; larger ones return at once, split or not.
-                cus = torch.cuda.get_device_properties(dev).multi_processor_count
-                self.looks = B <= 2 * cus
                 table, self.nsplit = _split_tables(parts)
                 self.split = torch.from_numpy(table).to(dev)
                 self.sws = _split_workspace(self.lib, self.nsplit, dev)
@@ -811,7 +807,7 @@ class RaggedGraph:
         if self.parts is not None:
             self.items.copy_(torch.from_numpy(_split_items(order, self.parts)))
         self.graph.replay()
-        if self.parts is not None and self.looks:
+        if self.parts is not None:
             _warn_unsolved(self.status)
         return RaggedResult(u=self.u, v=self.v, niter=self.niter, status=self.status,
                             err_first=self.e_first, err_last=self.e_last,

@@ -1,5 +1,4 @@
-"""Split point-cloud problems whose parts wait for a workgroup, and the calls
-that launch them without a host wait."""
+"""Split point-cloud problems whose parts wait for a workgroup."""
 
 import numpy as np
 import pytest
@@ -56,16 +55,6 @@ def test_a_split_solve_returns_without_a_wait():
     assert not before.query()
     torch.cuda.synchronize()
     assert torch.equal(got.u, want.u) and torch.equal(got.v, want.v)
-
-
-def test_a_split_graph_returns_before_its_replay_ends():
-    ns, ms, xs, ys, regs = _uneven(600)
-    G = ragged.RaggedGraph(ns, ms, 4, numItermax=4000, stopThr=0.0, cost="points",
-                           split=ragged.auto_plan(ns, ms))
-    assert G.parts is not None
-    G.solve(xs, ys, regs)
-    assert not torch.cuda.current_stream().query()
-    torch.cuda.synchronize()
 
 
 def test_the_automatic_split_leaves_full_batches_whole():
