@@ -84,12 +84,14 @@ int potamd_resident_wait_limit(int us);
  *    ot.batch stop, ot/batch/_utils.py:273-278), 1 = Frobenius norm (the
  *    multi-histogram knopp, ot/bregman/_sinkhorn.py:646-652, which runs the
  *    histograms as a batch sharing M through bstride = 0).
- * err_hist: float64 device array of err_cap entries, the reference's
- *    log["err"] (one value per check).
+ * err_hist: float64, err_cap entries in device memory or in pinned host memory
+ *    that the device can write, the reference's log["err"] (one value per
+ *    check); complete when the call returns.
  * threads, cols_per_thread, rows_per_block, prefetch (rows loaded ahead, 1
  *    or 2): tile shape, 0 = automatic.
- * host_ctrl: pinned host memory of >= 512 bytes used for asynchronous stop
- *    polling, or NULL (then each check synchronises).
+ * host_ctrl: pinned host memory of >= 512 bytes, or NULL (then each check
+ *    synchronises).  Copies and kernels of the call write their stop and its
+ *    outcome there; it belongs to one call at a time.
  * info (host, 4 ints): [0] niter (the reference's `ii`), [1] number of err
  *    values, [2] status, [3] iteration of a numerical stop.
  */
@@ -400,7 +402,7 @@ int potamd_mlp_fused(int mode, int rows, int seg_len, const void* inp, const flo
  * without materialising M; the reference's own lazy path is
  * empirical_sinkhorn(isLazy=True) (ot/bregman/_empirical.py:193-270).
  * Precision of the x . y^T term: */
-#define POTAMD_ONLINE_F32 0    /* fp32 MFMA */
+#define POTAMD_ONLINE_F32 0    /* fp32, as three bf16 parts on MFMA */
 #define POTAMD_ONLINE_BF16 1   /* bf16 MFMA, fp32 accumulation */
 #define POTAMD_ONLINE_BF16X3 2 /* bf16 hi + lo split, three MFMA products */
 #define POTAMD_ONLINE_FP8 3    /* fp8 e4m3 MFMA, per-point scale */

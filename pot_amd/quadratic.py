@@ -283,8 +283,8 @@ def solve_gromov_batch(C1, C2, reg=1e-2, a=None, b=None, loss="sqeuclidean", sym
         # log T - lin / reg, where lin = (1 - alpha) M + 2 alpha (constC - w S).
         # The products are taken from constC itself: the two may cancel, so
         # neither is scaled before (scaled by 2 alpha / reg first, the roundings
-        # of both stay: structures of 1000 + small integers, 1e-9 of the plan
-        # against 1e-14).
+        # of both stay: structures of 2000 + small integers, 5e-9 of the plan
+        # against 5e-14).
         lin0 = (1 - alpha) * Md
         w = -1.0 if symmetric else -0.5
         two_alpha = 2.0 * (alpha.item() if isinstance(alpha, torch.Tensor) else float(alpha))
