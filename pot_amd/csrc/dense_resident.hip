@@ -112,9 +112,9 @@ struct Choice {
 // element on the resident workgroups of a CU (4 clocks each), about 1100
 // clocks of reductions, divisions and barriers, and 3000 to 6000 clocks for an
 // exchange, more with more members (measured a whole iteration, 2.4 GHz: one
-// workgroup 0.9 us at 64 x 64, 1.6 at 100 x 120 and 2.3 at 200 x 120 in
-// float64; blocked 4.9 us at 300^2 (3 x 3), 6.3 at 1000 x 900, 7.5 at 2048^2
-// (16 x 16); the row sweep took 12, 12, 12, 13, 25 and 37 us).  So a problem
+// workgroup 1.1 us at 64 x 64, 1.8 at 100 x 120 and 2.3 at 200 x 120 in the
+// float64 log domain; blocked 4.9 us at 300^2 (3 x 3), 5.4 at 1000 x 900, 6.8 at
+// 2048^2 (16 x 16); the row sweep took 13, 13, 14, 15, 22 and 37 us).  So a problem
 // that fits one workgroup stays in one.
 // Of two tiles of one size (128 x 128 by eight waves or by four of twice the
 // elements) the fewer waves where there are more problems than CUs, as more such

@@ -52,9 +52,8 @@
 
 // (10 x 20: all of a CU's registers for K, 320 x 320 a workgroup, so that
 // 5120^2 float32 fits the chip; the rest spills, 0.2 to 0.3 KB a thread.
-// 5000 x 4999: 12.8 us an iteration in the scaling domain and 34.8 in the log
-// domain, against 61 and 64 on the row sweep (36 and 38 where rows are
-// 16-byte aligned).)
+// 5000 x 4999: 12.3 us an iteration in the scaling domain and 36 in the log
+// domain, against 49 on the row sweep.)
 #define POTAMD_TILES_F32(X) \
   X(4, 2, 4) X(4, 4, 4) X(8, 4, 8) X(4, 8, 8) X(8, 8, 8) X(8, 4, 16) X(8, 8, 16) X(8, 10, 20)
 #define POTAMD_TILES_F64(X) X(4, 2, 4) X(4, 4, 4) X(8, 2, 8) X(8, 4, 8) X(4, 8, 8) X(8, 8, 8) X(8, 4, 16)
