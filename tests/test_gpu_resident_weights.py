@@ -1,0 +1,30 @@
+"""Weights that leave no plan or a meaningless one, in the register-resident
+solves: outcomes are the row sweep's and the oracle's."""
+
+import pytest
+import torch
+
+from pot_amd import _lib, _solve
+
+pytestmark = pytest.mark.gpu
+
+F32, F64 = torch.float32, torch.float64
+
+
+@pytest.mark.parametrize("dtype", [F64, F32])
+@pytest.mark.parametrize("n,m", [(5, 4), (60, 50), (400, 360)])
+@pytest.mark.parametrize("order", [_lib.COL_FIRST, _lib.ROW_FIRST])
+def test_no_weight_in_any_column(n, m, order, dtype):
+    g = torch.Generator("cuda").manual_seed(n)
+    M = torch.rand(1, n, m, generator=g, device="cuda", dtype=dtype)
+    a = torch.full((1, n), 1.0 / n, device="cuda", dtype=F64)
+    b = torch.zeros((1, m), device="cuda", dtype=F64)
+    assert _lib.load().potamd_dense_resident(_lib.F32 if dtype == F32 else _lib.F64, 1, n, m)
+    kw = dict(domain=_lib.LOG, order=order, max_iter=20, stop_thr=1e-9)
+    tile = (256, 4, 0, 1) if m > 128 else (64, 4, 0, 1) if dtype == F32 else (64, 2, 0, 1)
+    want = _solve.dense_solve(M, a, b, torch.zeros_like(a), torch.zeros_like(b), 0.05, tile=tile,
+                              **kw)
+    got = _solve.dense_solve(M, a, b, torch.zeros_like(a), torch.zeros_like(b), 0.05, **kw)
+    assert (got.status, got.niter, got.errs) == (want.status, want.niter, want.errs)
+    for x, y in ((got.u, want.u), (got.v, want.v)):
+        torch.testing.assert_close(x, y, rtol=0, atol=0, equal_nan=True)
