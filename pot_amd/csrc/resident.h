@@ -813,7 +813,7 @@ __global__ __launch_bounds__(64 * W, 2) void resident_kernel(ResidentArgs A) {
         if (b_t == 0.0 ? c != c : !(g_prev * c >= kFloor))
           atomicOr(&events, 2);
         else if (b_t != 0.0 && off_range(g_t))
-          atomicOr(&events, (!__builtin_isfinite(g_t) || g_t == 0.0) ? 2 : 1);
+          atomicOr(&events, (!__builtin_isfinite(g_t) || !(g_t > 0.0)) ? 2 : 1);
       } else if (c == 0.0 || !__builtin_isfinite(c) || !__builtin_isfinite(g_t)) {
         atomicOr(&events, 2);  // (a row scaling that is not finite makes every c so)
       }

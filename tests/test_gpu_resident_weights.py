@@ -28,3 +28,19 @@ def test_no_weight_in_any_column(n, m, order, dtype):
     assert (got.status, got.niter, got.errs) == (want.status, want.niter, want.errs)
     for x, y in ((got.u, want.u), (got.v, want.v)):
         torch.testing.assert_close(x, y, rtol=0, atol=0, equal_nan=True)
+
+
+@pytest.mark.parametrize("dtype", [F64, F32])
+@pytest.mark.parametrize("B,n,m", [(1, 5, 4), (3, 60, 50), (1, 400, 360), (2100, 20, 33)])
+def test_negative_column_weight_is_refused(B, n, m, dtype):
+    """Its logarithm is no number: the log domain raises, rows first too."""
+    g = torch.Generator("cuda").manual_seed(n)
+    M = torch.rand(B, n, m, generator=g, device="cuda", dtype=dtype)
+    a = torch.full((B, n), 1.0 / n, device="cuda", dtype=F64)
+    b = torch.full((B, m), 1.0 / m, device="cuda", dtype=F64)
+    b[B // 2, 1] = -0.1
+    for order in (_lib.COL_FIRST, _lib.ROW_FIRST):
+        for iters in (1, 25):
+            with pytest.raises(_lib.LibraryError):
+                _solve.dense_solve(M, a, b, torch.zeros_like(a), torch.zeros_like(b), 0.05,
+                                   domain=_lib.LOG, order=order, max_iter=iters, stop_thr=0.0)
