@@ -700,7 +700,7 @@ __global__ __launch_bounds__(64 * W, 2) void resident_kernel(ResidentArgs A) {
         // (One lane of a wave raises the flag: where most scalings pass tau, an
         // atomic of each took 1 us an iteration.  1000 x 900 float64 with an
         // absorption in every one 12.6 us, 11.9 now; 1524 x 661 15.8 and 14.1.)
-        if (STAB && __any(f_l > A.tau) && lane == 0) atomicOr(&events, 8);
+        if (STAB && __any(fabs(f_l) > A.tau) && lane == 0) atomicOr(&events, 8);
         if (LOG) {
           if (!live) f_l = 0.0;
           slow = __any(live && off_range(S));  // (a wave has its rows to itself)
@@ -819,7 +819,7 @@ __global__ __launch_bounds__(64 * W, 2) void resident_kernel(ResidentArgs A) {
       }
       gsh[tid] = (R)g_t;
     }
-    if (STAB && __any(cown && __builtin_isfinite(c) && g_t > A.tau) && lane == 0)
+    if (STAB && __any(cown && __builtin_isfinite(c) && fabs(g_t) > A.tau) && lane == 0)
       atomicOr(&events, 20 - over_last);
     __syncthreads();
     over_last = 20 - over_last;

@@ -1,9 +1,14 @@
 """Weights that leave no plan or a meaningless one, in the register-resident
 solves: outcomes are the row sweep's and the oracle's."""
 
+import warnings
+
+import numpy as np
 import pytest
 import torch
 
+import oracle.stabilized as ostab
+import pot_amd
 from pot_amd import _lib, _solve
 
 pytestmark = pytest.mark.gpu
@@ -44,3 +49,29 @@ def test_negative_column_weight_is_refused(B, n, m, dtype):
             with pytest.raises(_lib.LibraryError):
                 _solve.dense_solve(M, a, b, torch.zeros_like(a), torch.zeros_like(b), 0.05,
                                    domain=_lib.LOG, order=order, max_iter=iters, stop_thr=0.0)
+
+
+def _both(a, b, M, reg, **kw):
+    with warnings.catch_warnings(record=True) as W:
+        warnings.simplefilter("always")
+        P, lg = pot_amd.sinkhorn(*(torch.tensor(x, device="cuda") for x in (a, b, M)), reg,
+                                 method="sinkhorn_stabilized", log=True, warn=False, **kw)
+        got = [str(w.message) for w in W]
+    with warnings.catch_warnings(record=True) as W, np.errstate(all="ignore"):
+        warnings.simplefilter("always")
+        Q, lo = ostab.sinkhorn_stabilized(a, b, M, reg, log=True, warn=False, **kw)
+        want = [str(w.message) for w in W]
+    assert got == want and lg["n_iter"] == lo["n_iter"]
+    np.testing.assert_allclose(P.cpu().numpy(), Q, rtol=1e-10, atol=1e-18, equal_nan=True)
+    return want
+
+
+@pytest.mark.parametrize("n,m", [(6, 5), (60, 50), (400, 360)])
+def test_stabilized_negative_weight_is_over_tau_too(n, m):
+    """max |u| decides about absorption, whose logarithm then is no number."""
+    rng = np.random.default_rng(n)
+    a, b = rng.dirichlet(np.ones(n)), rng.dirichlet(np.ones(m))
+    a[0] = -2.0
+    M = rng.random((n, m))
+    for iters in (1, 2, 7):
+        _both(a, b, M, 0.2, numItermax=iters, tau=abs(a[0]))
