@@ -779,12 +779,12 @@ __global__ __launch_bounds__(64 * W, 2) void resident_kernel(ResidentArgs A) {
         ++n_err;
         next_check += A.period;
       }
-      if (last_err <= A.stop_thr) {
-        status = kConverged;
-        niter = it;
-        break;
-      }
-      if (it >= A.max_iter - 1) {
+      const bool stop = last_err <= A.stop_thr;
+      if (stop || it >= A.max_iter - 1) {
+        // (a row scaling that is no number makes every column sum so; the pair
+        // before it is the outcome then)
+        if (__syncthreads_or(cown && c != c)) return abandon();
+        if (stop) status = kConverged;
         niter = it;
         break;
       }

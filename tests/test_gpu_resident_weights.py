@@ -75,3 +75,14 @@ def test_stabilized_negative_weight_is_over_tau_too(n, m):
     M = rng.random((n, m))
     for iters in (1, 2, 7):
         _both(a, b, M, 0.2, numItermax=iters, tau=abs(a[0]))
+
+
+@pytest.mark.parametrize("n,m", [(6, 5), (60, 50), (400, 360)])
+@pytest.mark.parametrize("iters", [1, 3])
+def test_stabilized_row_without_weight_or_kernel(n, m, iters):
+    """0 / 0 in a row's scaling, in the last iteration as in an earlier one."""
+    rng = np.random.default_rng(n)
+    a, b = rng.dirichlet(np.ones(n)), rng.dirichlet(np.ones(m))
+    M = rng.random((n, m))
+    a[1], M[1] = 0.0, 1e3
+    assert _both(a, b, M, 0.05, numItermax=iters) == ["Numerical errors at iteration 0"]
