@@ -604,6 +604,16 @@ __global__ __launch_bounds__(64 * W, 2) void resident_kernel(ResidentArgs A) {
     return hi - ((1023u - kDrift) << 20) > ((2u * kDrift) << 20);
   };
 
+  // Whether this thread's column cannot be updated from its sum c: no number, a
+  // mass below the trusted range, or a scaling that the row sweep reports.
+  auto no_update = [&](double c) -> bool {
+    if (!cown) return false;
+    const double g = b_t / c;
+    if (LOG)
+      return b_t == 0.0 ? c != c : !(g_t * c >= kFloor) || !__builtin_isfinite(g) || !(g > 0.0);
+    return c == 0.0 || !__builtin_isfinite(c) || !__builtin_isfinite(g);
+  };
+
   // Square root of the problems' summed squared errors, joint over the batch.
   // Returns -1 where the launch ends here (segment) or the wait gave up.
   auto joint_error = [&](double e2, int parts, bool publish, int me) -> double {
@@ -792,12 +802,18 @@ __global__ __launch_bounds__(64 * W, 2) void resident_kernel(ResidentArgs A) {
     if (!STAB && check_cols && it == next_check) {
       const double d = g_t * c - b_t;
       const double err = joint_error(cown ? d * d : 0.0, GC, I == 0, J);
-      if (A.segment) break;
+      // (the update that follows decides first: what it gives up on is neither
+      // converged nor the last state)
+      if (A.segment) {
+        if (__syncthreads_or(no_update(c))) return abandon();
+        break;
+      }
       if (dead) return abandon();
       if (!A.each && blockIdx.x == 0 && tid == 0 && n_err < A.err_cap) A.err_hist[n_err] = err;
       ++n_err;
       next_check += 10;
       if (err < A.stop_thr) {
+        if (__syncthreads_or(no_update(c))) return abandon();
         status = kConverged;
         niter = it;
         break;
@@ -806,17 +822,12 @@ __global__ __launch_bounds__(64 * W, 2) void resident_kernel(ResidentArgs A) {
     check_cols = !row_first;
     g_prev = g_t;
     if (cown) {
-      g_t = b_t / c;
-      if (LOG) {
-        if (b_t == 0.0)
-          g_t = 0.0;
-        if (b_t == 0.0 ? c != c : !(g_prev * c >= kFloor))
-          atomicOr(&events, 2);
-        else if (b_t != 0.0 && off_range(g_t))
-          atomicOr(&events, (!__builtin_isfinite(g_t) || !(g_t > 0.0)) ? 2 : 1);
-      } else if (c == 0.0 || !__builtin_isfinite(c) || !__builtin_isfinite(g_t)) {
-        atomicOr(&events, 2);  // (a row scaling that is not finite makes every c so)
-      }
+      const bool none = no_update(c);  // (a row scaling that is not finite makes every c so)
+      g_t = LOG && b_t == 0.0 ? 0.0 : b_t / c;
+      if (none)
+        atomicOr(&events, 2);
+      else if (LOG && b_t != 0.0 && off_range(g_t))
+        atomicOr(&events, 1);
       gsh[tid] = (R)g_t;
     }
     if (STAB && __any(cown && __builtin_isfinite(c) && fabs(g_t) > A.tau) && lane == 0)

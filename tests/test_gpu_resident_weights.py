@@ -86,3 +86,35 @@ def test_stabilized_row_without_weight_or_kernel(n, m, iters):
     M = rng.random((n, m))
     a[1], M[1] = 0.0, 1e3
     assert _both(a, b, M, 0.05, numItermax=iters) == ["Numerical errors at iteration 0"]
+
+
+def _outcome(M, a, b, tile=None, **kw):
+    n, m = M.shape[1:]
+    scal = kw["domain"] == _lib.SCALING
+    u0 = torch.full_like(a, 1.0 / n) if scal else torch.zeros_like(a)
+    v0 = torch.full_like(b, 1.0 / m) if scal else torch.zeros_like(b)
+    try:
+        r = _solve.dense_solve(M, a, b, u0, v0, 0.05, tile=tile, order=_lib.COL_FIRST, **kw)
+    except _lib.LibraryError as e:
+        return str(e)
+    return r.status, r.niter, r.bad_iter, len(r.errs)
+
+
+@pytest.mark.parametrize("dtype", [F64, F32])
+@pytest.mark.parametrize("B,n,m", [(1, 5, 4), (4, 60, 50), (1, 400, 360), (2100, 9, 7)])
+def test_update_after_a_check_decides_first(B, n, m, dtype):
+    """Iterations that check and end (converged, or the last) with a column that
+    cannot be updated: masses below the trusted range, weights that are no number."""
+    g = torch.Generator("cuda").manual_seed(n)
+    M = torch.rand(B, n, m, generator=g, device="cuda", dtype=dtype)
+    a = torch.full((B, n), 1.0 / n, device="cuda", dtype=F64)
+    b = torch.full((B, m), 1.0 / m, device="cuda", dtype=F64)
+    nan = a.clone()
+    nan[B // 2, 0] = float("nan")
+    tile = (256, 4, 0, 1) if m > 128 else (64, 4, 0, 1) if dtype == F32 else (64, 2, 0, 1)
+    for domain in (_lib.LOG, _lib.SCALING):
+        for iters, stop in ((1, 0.0), (32, 1e-7)):
+            kw = dict(domain=domain, max_iter=iters, stop_thr=stop,
+                      err_norm=int(domain == _lib.SCALING))
+            for x, y in ((a * 1e-302, b * 1e-302), (nan, b), (a, b)):
+                assert _outcome(M, x, y, **kw) == _outcome(M, x, y, tile=tile, **kw)
